@@ -6,6 +6,7 @@
 #include <type_traits>
 
 #include "pa_common.hpp"
+#include "pa_internal.hpp"
 #include "../../include/pa_dense.h"
 
 namespace pa {
@@ -829,58 +830,7 @@ __global__ __launch_bounds__(kArgmaxThreads) void argmax_kernel(int64_t* __restr
 }
 
 
-// ---------------------------------------------------------------------------
-// Prefill-sized linear layer: Y[M, N] = X[M, K] · W[N, K]ᵀ (bf16, f32
-// accumulation) for batches of many rows (prompt chunks), where the
-// arithmetic, not the weight stream, bounds the work.
-//
-// Workgroup = WM x WN wavefronts; wavefront (wm, wn) computes TM x TN tiles
-// of 32 x 32 (v_mfma_f32_32x32x16_bf16), so the workgroup tile is
-// BM = 32 WM TM rows x BN = 32 WN TN weight rows, K in steps of BK.  Each
-// step's X and W tiles are copied HBM -> LDS with global_load_lds (no
-// register staging) into one of two buffers, one step ahead of use; the
-// grid is persistent (the LDS-resident workgroups of the GPU), and a
-// workgroup's steps run as one sequence over its tiles, so the next tile's
-// first copy is in flight during a tile's epilogue.
-// Operand reads: lane l = 32 g + n takes row n of a 32-row tile, k 8 g ..
-// 8 g + 7 of the MFMA's 16 (one 16-byte LDS read, which feeds TN or TM
-// MFMAs); the tiles' rows (2 BK bytes) hold their 16-byte k chunks
-// XOR-swizzled by the row's position above the rows that share 256 bytes
-// (chunk position ch ^ ((r / (256 / 2 BK)) % (BK / 8))), so the 16 rows a
-// read serves at once hit 16 distinct bank slots.
-// The MFMAs compute the transposed tile (W rows x X rows: A = W, B = X), so
-// lane (n, g) holds X row n and, in register r, output column
-// 8 (r / 4) + 4 g + r % 4: four consecutive columns per 8-byte store.
-// Epilogues (EPI): 0 none; 1 + bias[n]; 2 SwiGLU over a fused gate|up
-// weight [2 N, K]: the workgroup's BN weight rows are gate rows a0 ..
-// a0 + BN/2 - 1 then the up rows N + a0 .. (a0 = BN/2 x the column tile),
-// wavefront wn takes its TN/2 gate tiles and the matching up tiles, and
-// out[m][a] = silu(bf16(g)) * bf16(u) (the exponential
-// __expf, the reciprocal v_rcp_f32); with add_out the result is added into
-// out (out = bf16(out + bf16(y))).  Rows past M read row M - 1, weight rows
-// past N (EPI 0 / 1: N need not fill the last tile) read row N - 1, and
-// neither is stored.
-#ifndef PA_GEMM_BIG_BK
-#define PA_GEMM_BIG_BK 64
-#define PA_GEMM_BIG_S 2
-#define PA_GEMM_SMALL_BK 64
-#define PA_GEMM_SMALL_S 2
-#endif
 constexpr int kSkinnyMaxRows = 64;
-// HBM -> LDS copy of 16 bytes per lane (lane l's bytes land at lds + 16 l),
-// written out in assembly: with the builtin, the compiler cannot tell that
-// the operand reads which follow use the other LDS buffer, and makes them
-// wait for the copy (vmcnt(0) right after every copy, so no copy overlapped
-// any compute).  The kernel orders copies and reads itself (vmcnt(0) and a
-// barrier at the top of every step).
-__device__ inline void lds_copy16(const void* src, void* lds) {
-  const uint32_t m0 = __builtin_amdgcn_readfirstlane(
-      (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds);
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off"
-               :
-               : "v"(src), "s"(m0)
-               : "memory", "m0");
-}
 // Compute units of the current device (cached per device).
 int gemm_compute_units() {
   static int cached[64] = {0};
@@ -894,260 +844,8 @@ int gemm_compute_units() {
     cached[dev] = n;
   }
   return cached[dev];
-}  // pa_linear's skinny kernel up to here
-constexpr int kGemmKMultiple = 64;  // K the tiled kernel takes: a multiple of this
-constexpr int kGemmGroupM = 4;  // row tiles per group of the tile order
-template <int EPI, int WM, int WN, int TM, int TN, int BK, int S>
-__global__ __launch_bounds__(64 * WM * WN) void gemm_tiled_kernel(
-    uint16_t* __restrict__ out, const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
-    const uint16_t* __restrict__ bias, int M, int N, int K, int add_out, int ntm, int ntn) {
-  constexpr int NW = WM * WN;
-  constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
-  static_assert(kGemmKMultiple % BK == 0, "K steps");
-  constexpr int RB = BK * 2;           // bytes per tile row
-  constexpr int RPC = 1024 / RB;       // rows per 1 KB copy chunk
-  constexpr int LPR = RB / 16;         // lanes (16-byte chunks) per row
-  constexpr int CA = BM / RPC / NW, CB = BN / RPC / NW;  // copy chunks per wavefront
-  static_assert(CA * NW * RPC == BM && CB * NW * RPC == BN && (EPI != 2 || TN % 2 == 0),
-                "tiles");
-  __shared__ __attribute__((aligned(1024))) uint8_t lds_a[S][BM * RB];
-  __shared__ __attribute__((aligned(1024))) uint8_t lds_b[S][BN * RB];
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wm = wave / WN, wn = wave % WN;
-  const int n = lane & 31, g = lane >> 5;
-  // Persistent grid, tile order: workgroups are dealt round-robin to the 8
-  // XCDs; XCD x takes the contiguous range [x per_xcd, (x + 1) per_xcd) of
-  // the logical order, its workgroups (slots) taking every nslot-th tile of
-  // it, so the tiles in flight on an XCD are neighbours in the order.  The
-  // order goes through groups of kGemmGroupM row tiles, column tiles outer
-  // within a group, so those workgroups share X rows and W rows in the
-  // XCD's L2.
-  const int total = ntm * ntn, per_xcd = (total + 7) / 8;
-  const int xcd = (int)(blockIdx.x % 8), slot = (int)(blockIdx.x / 8);
-  const int nslot = (int)(gridDim.x / 8);
-  const int lo = xcd * per_xcd, hi = min(total, lo + per_xcd);
-  if (lo + slot >= hi) return;
-  const int my_tiles = (hi - 1 - lo - slot) / nslot + 1;
-  auto tile_origin = [&](int i, int& m0, int& c0) __attribute__((always_inline)) {
-    const int L = lo + slot + i * nslot;
-    const int grp = L / (kGemmGroupM * ntn), first_m = grp * kGemmGroupM;
-    const int gsz = min(kGemmGroupM, ntm - first_m);
-    const int r = L % (kGemmGroupM * ntn);
-    m0 = (first_m + r % gsz) * BM;
-    c0 = (r / gsz) * (EPI == 2 ? BN / 2 : BN);  // first output column
-  };
-  auto swz = [](int r) -> int { return (r / (256 / RB)) % LPR; };
-  // this wavefront's copies: RPC rows per 1 KB chunk; lane l fills chunk
-  // position l % LPR of row l / LPR, i.e. source chunk (l % LPR) ^ swz(row)
-  int xr[CA], wr[CB], xch[CA], wch[CB];
-#pragma unroll
-  for (int i = 0; i < CA; ++i) {
-    xr[i] = (CA * wave + i) * RPC + lane / LPR;
-    xch[i] = ((lane % LPR) ^ swz(xr[i])) * 8;
-  }
-#pragma unroll
-  for (int i = 0; i < CB; ++i) {
-    wr[i] = (CB * wave + i) * RPC + lane / LPR;
-    wch[i] = ((lane % LPR) ^ swz(wr[i])) * 8;
-  }
-  // copies of step kt of the tile whose source rows are xs / ws into
-  // buffer BUF; the rows change only per tile (set_sources)
-  const uint16_t* xs[CA];
-  const uint16_t* ws[CB];
-  auto set_sources = [&](int i) __attribute__((always_inline)) {
-    int m0, c0;
-    tile_origin(i, m0, c0);
-#pragma unroll
-    for (int u = 0; u < CA; ++u) xs[u] = x + (int64_t)min(m0 + xr[u], M - 1) * K + xch[u];
-#pragma unroll
-    for (int u = 0; u < CB; ++u) {
-      const int r = wr[u];
-      const int row = EPI == 2 ? (r < BN / 2 ? c0 + r : N + c0 + r - BN / 2) : min(c0 + r, N - 1);
-      ws[u] = w + (int64_t)row * K + wch[u];
-    }
-  };
-  auto issue = [&](int kt, int buf) __attribute__((always_inline)) {
-    uint8_t* la = lds_a[buf];
-    uint8_t* lb = lds_b[buf];
-#pragma unroll
-    for (int u = 0; u < CA; ++u)
-      lds_copy16(xs[u] + kt * BK, &la[(CA * wave + u) * 1024]);
-#pragma unroll
-    for (int u = 0; u < CB; ++u)
-      lds_copy16(ws[u] + kt * BK, &lb[(CB * wave + u) * 1024]);
-  };
-  // LDS rows of this wavefront's operand tiles (SwiGLU: gate tiles, then
-  // the matching up tiles)
-  int arow[TM], brow[TN];
-#pragma unroll
-  for (int t = 0; t < TM; ++t) arow[t] = (wm * TM + t) * 32 + n;
-#pragma unroll
-  for (int t = 0; t < TN; ++t)
-    brow[t] = EPI == 2 ? (t < TN / 2 ? (wn * TN / 2 + t) * 32 + n
-                                     : BN / 2 + (wn * TN / 2 + t - TN / 2) * 32 + n)
-                       : (wn * TN + t) * 32 + n;
-  f32x16 acc[TM][TN];
-#pragma unroll
-  for (int a = 0; a < TM; ++a)
-#pragma unroll
-    for (int b = 0; b < TN; ++b)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[a][b][i] = 0.f;
-  // epilogue of the tile at (m0, c0)
-  auto store_tile = [&](int m0, int c0) __attribute__((always_inline)) {
-  // epilogue: acc[a][b] is the transposed tile (W rows x X rows), so lane
-  // (n, g) holds X row n and, in registers 4 q .. 4 q + 3, the four
-  // consecutive output columns 8 q + 4 g .. 8 q + 4 g + 3 (one 8-byte store)
-  const bool vec = N % 4 == 0;
-#pragma unroll
-  for (int a = 0; a < TM; ++a) {
-    const int row = m0 + (wm * TM + a) * 32 + n;
-    if (row >= M) continue;
-    uint16_t* orow = out + (int64_t)row * N;
-    if constexpr (EPI == 2) {
-#pragma unroll
-      for (int b = 0; b < TN / 2; ++b)
-#pragma unroll
-        for (int qd = 0; qd < 4; ++qd) {
-          const int col = c0 + (wn * TN / 2 + b) * 32 + 8 * qd + 4 * g;
-          uint16_t v[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float gg = (float)(__bf16)acc[a][b][4 * qd + e];
-            const float uu = (float)(__bf16)acc[a][b + TN / 2][4 * qd + e];
-            v[e] = __builtin_bit_cast(
-                uint16_t, (__bf16)(gg * __builtin_amdgcn_rcpf(1.0f + __expf(-gg)) * uu));
-          }
-          *reinterpret_cast<uint64_t*>(orow + col) = *reinterpret_cast<const uint64_t*>(v);
-        }
-    } else {
-      // every load of the epilogue is issued before any of its values is
-      // used (bias once for the tile, the residual row's values per row),
-      // so the round trips overlap instead of following one another
-      float bv[TN][4][4];
-#pragma unroll
-      for (int b = 0; b < TN; ++b)
-#pragma unroll
-        for (int qd = 0; qd < 4; ++qd)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int col = c0 + (wn * TN + b) * 32 + 8 * qd + 4 * g + e;
-            bv[b][qd][e] = EPI == 1 ? bf16_bits_to_f32(bias[min(col, N - 1)]) : 0.f;
-          }
-      uint64_t ow[TN][4];
-      if (add_out && vec) {
-#pragma unroll
-        for (int b = 0; b < TN; ++b)
-#pragma unroll
-          for (int qd = 0; qd < 4; ++qd) {
-            const int col = c0 + (wn * TN + b) * 32 + 8 * qd + 4 * g;
-            ow[b][qd] = col < N ? *reinterpret_cast<const uint64_t*>(orow + col) : 0;
-          }
-      }
-#pragma unroll
-      for (int b = 0; b < TN; ++b)
-#pragma unroll
-        for (int qd = 0; qd < 4; ++qd) {
-          const int col = c0 + (wn * TN + b) * 32 + 8 * qd + 4 * g;
-          if (col >= N) continue;
-          float y[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) y[e] = acc[a][b][4 * qd + e] + bv[b][qd][e];
-          if (vec) {
-            uint16_t v[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              float t = y[e];
-              if (add_out)
-                t = bf16_bits_to_f32((uint16_t)(ow[b][qd] >> (16 * e))) +
-                    bf16_bits_to_f32(f32_to_bf16_bits(t));
-              v[e] = f32_to_bf16_bits(t);
-            }
-            *reinterpret_cast<uint64_t*>(orow + col) = *reinterpret_cast<const uint64_t*>(v);
-          } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              if (col + e >= N) continue;
-              float t = y[e];
-              if (add_out) t = bf16_bits_to_f32(orow[col + e]) + bf16_bits_to_f32(f32_to_bf16_bits(t));
-              orow[col + e] = f32_to_bf16_bits(t);
-            }
-          }
-        }
-    }
-  }
-  };
-  // The workgroup's steps run as one sequence over its tiles (step gs =
-  // step gs % nk of tile gs / nk, in buffer gs % 2), the copy of step gs + 1
-  // issued before step gs is computed -- across tile boundaries too, so the
-  // next tile's first copy is in flight during the epilogue.
-  const int nk = K / BK, nsteps = my_tiles * nk;
-  // Copies run S - 1 steps ahead: before step gs computes, the copies of
-  // steps gs + 1 .. gs + S - 2 may still be in flight (CA + CB loads each).
-  constexpr int PER = CA + CB;
-  static_assert(PER * (S - 2) <= 63 && S >= 2 && S <= 4, "vmcnt range");
-  int cur = 0;      // tile of the step being computed
-  int iss = 0;      // next step to copy, and its tile / step within the tile
-  int iss_tile = 0, iss_kt = 0;
-  set_sources(0);
-  auto issue_next = [&]() __attribute__((always_inline)) {
-    if (iss_kt == nk) {  // the step starts the next tile
-      ++iss_tile;
-      iss_kt = 0;
-      set_sources(iss_tile);
-    }
-    issue(iss_kt, iss % S);
-    ++iss;
-    ++iss_kt;
-  };
-  for (int t = 0; t < S - 1 && t < nsteps; ++t) issue_next();
-  for (int gs = 0; gs < nsteps; ++gs) {
-    const int kt = gs - cur * nk;
-    const int ahead = iss - 1 - gs;  // copies of later steps in flight
-    if (ahead >= 2)
-      __builtin_amdgcn_s_waitcnt(0x0F70 | ((2 * PER) & 0xF) | (((2 * PER) >> 4) << 14));
-    else if (ahead == 1)
-      __builtin_amdgcn_s_waitcnt(0x0F70 | (PER & 0xF) | ((PER >> 4) << 14));
-    else
-      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-    // step gs has landed for every wavefront, and every wavefront is done
-    // with step gs - 1's buffer, which the next copy reuses
-    __syncthreads();
-    if (iss < nsteps) issue_next();
-    const uint8_t* at = lds_a[gs % S];
-    const uint8_t* bt = lds_b[gs % S];
-#pragma unroll
-    for (int s = 0; s < BK / 16; ++s) {
-      bf16x8 af[TM], bfr[TN];
-#pragma unroll
-      for (int t = 0; t < TM; ++t)
-        af[t] = *reinterpret_cast<const bf16x8*>(at + arow[t] * RB +
-                                                 (((2 * s + g) ^ swz(arow[t])) * 16));
-#pragma unroll
-      for (int t = 0; t < TN; ++t)
-        bfr[t] = *reinterpret_cast<const bf16x8*>(bt + brow[t] * RB +
-                                                  (((2 * s + g) ^ swz(brow[t])) * 16));
-#pragma unroll
-      for (int a = 0; a < TM; ++a)
-#pragma unroll
-        for (int b = 0; b < TN; ++b)
-          acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[b], af[a], acc[a][b], 0, 0, 0);
-    }
-    if (kt == nk - 1) {
-      int m0, c0;
-      tile_origin(cur, m0, c0);
-      store_tile(m0, c0);
-#pragma unroll
-      for (int a = 0; a < TM; ++a)
-#pragma unroll
-        for (int b = 0; b < TN; ++b)
-#pragma unroll
-          for (int q = 0; q < 16; ++q) acc[a][b][q] = 0.f;
-      ++cur;
-    }
-  }
 }
+constexpr int kGemmKMultiple = 64;  // K the tiled kernel takes: a multiple of this
 
 }  // namespace
 }  // namespace pa
@@ -1313,58 +1011,9 @@ extern "C" int32_t pa_linear(void* out, const void* x, const void* weight, const
   PA_REQUIRE(tiled || out_features % 16 == 0, PA_ERR_UNSUPPORTED,
              "pa_linear: out_features %d not a multiple of 16", out_features);
   if (tiled) {
-    // Large outputs: 256 x 256 workgroup tiles (8 wavefronts of 64 x 128:
-    // each operand read feeds 4 or 2 MFMAs); otherwise 128 x 128 (4
-    // wavefronts of 64 x 64), which keeps small projections spread over
-    // more workgroups.
-    hipStream_t s = (hipStream_t)stream;
-    const int add = (flags & PA_LINEAR_ADD_OUT) ? 1 : 0;
-    auto* o = (uint16_t*)out;
-    auto* xx = (const uint16_t*)x;
-    auto* ww = (const uint16_t*)weight;
-    auto* bb = (const uint16_t*)bias;
-    const int wcols = act == PA_ACT_SILU_MUL ? 2 * out_features : out_features;
-    const bool big = (long long)((rows + 255) / 256) * ((wcols + 255) / 256) >= 256 &&
-                     (act != PA_ACT_SILU_MUL || out_features % 128 == 0);
-    auto launch = [&](auto wmc, auto wnc, auto tmc, auto tnc) -> int32_t {
-      constexpr int WM_ = decltype(wmc)::value, WN_ = decltype(wnc)::value;
-      constexpr int TM_ = decltype(tmc)::value, TN_ = decltype(tnc)::value;
-      // K steps of 64 through two LDS buffers (measured at the config-5
-      // shapes against steps of 32 through 2, 3 or 4 buffers: equal for the
-      // 256 x 256 tiles, 28.6 vs 33.6-36.4 us for the 128 x 128 ones)
-      constexpr int BK_ = WM_ * WN_ == 8 ? PA_GEMM_BIG_BK : PA_GEMM_SMALL_BK;
-      constexpr int S_ = WM_ * WN_ == 8 ? PA_GEMM_BIG_S : PA_GEMM_SMALL_S;
-      constexpr int WPC = WM_ * WN_ == 8 ? 1 : 2;  // workgroups per CU (LDS)
-      static_assert(WPC == 1 || WPC == 2, "");
-      constexpr int BM_ = 32 * WM_ * TM_, BN_ = 32 * WN_ * TN_;
-      const int ntn = act == PA_ACT_SILU_MUL ? out_features / (BN_ / 2)
-                                             : (out_features + BN_ - 1) / BN_;
-      const int ntm = (rows + BM_ - 1) / BM_;
-      PA_REQUIRE((long long)ntm * ntn < (1ll << 30), PA_ERR_UNSUPPORTED, "pa_linear: %d rows",
-                 rows);
-      const int per_xcd = (ntm * ntn + 7) / 8;
-      // persistent for the large tiles (one workgroup per CU: its next
-      // tile's first copy overlaps the epilogue); a workgroup per tile for
-      // the small ones (two per CU: one's epilogue overlaps the other's loop)
-      const dim3 grid(8 * (WPC == 1 ? std::max(1, std::min(per_xcd, gemm_compute_units() / 8))
-                                    : per_xcd));
-      if (act == PA_ACT_SILU_MUL)
-        gemm_tiled_kernel<2, WM_, WN_, TM_, TN_, BK_, S_><<<grid, 64 * WM_ * WN_, 0, s>>>(
-            o, xx, ww, nullptr, rows, out_features, in_features, 0, ntm, ntn);
-      else if (bias)
-        gemm_tiled_kernel<1, WM_, WN_, TM_, TN_, BK_, S_><<<grid, 64 * WM_ * WN_, 0, s>>>(
-            o, xx, ww, bb, rows, out_features, in_features, add, ntm, ntn);
-      else
-        gemm_tiled_kernel<0, WM_, WN_, TM_, TN_, BK_, S_><<<grid, 64 * WM_ * WN_, 0, s>>>(
-            o, xx, ww, nullptr, rows, out_features, in_features, add, ntm, ntn);
-      return PA_OK;
-    };
-    using I1 = std::integral_constant<int, 1>;
-    using I2 = std::integral_constant<int, 2>;
-    using I4 = std::integral_constant<int, 4>;
-    const int32_t rc = big ? launch(I4{}, I2{}, I2{}, I4{}) : launch(I2{}, I2{}, I2{}, I2{});
-    if (rc != PA_OK) return rc;
-    return check_launch("pa_linear");
+    return launch_gemm(out, x, weight, bias, rows, out_features, in_features,
+                       act == PA_ACT_SILU_MUL, (flags & PA_LINEAR_ADD_OUT) != 0,
+                       (hipStream_t)stream);
   }
   PA_REQUIRE((rows + 31) / 32 <= 65535, PA_ERR_UNSUPPORTED, "pa_linear: %d rows", rows);
   // A wide projection of one batch tile over packed weights (the LM head):

@@ -36,6 +36,13 @@ PA_HIDDEN int32_t launch_quant_read(const float* k_cache, const float* v_cache,
                                     const float* scales, const int32_t* block_ids, int seq_len,
                                     int H, int D, float* out_k, float* out_v, hipStream_t stream);
 
+// pa_linear for batches of many rows over a row-major weight (gemm.hip):
+// in_features a multiple of 64; silu: weight [2 out_features, in_features],
+// gate rows first.
+PA_HIDDEN int32_t launch_gemm(void* out, const void* x, const void* weight, const void* bias,
+                              int rows, int out_features, int in_features, bool silu,
+                              bool add_out, hipStream_t stream);
+
 // pa_decode / pa_prefill with q rows q_row elements apart (a view of a fused
 // QKV projection output); pa_batch_attention's path.
 PA_HIDDEN int32_t decode_strided(void* out, const void* q, int64_t q_row, const void* k_cache,
