@@ -26,6 +26,7 @@ namespace {
 
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kNegBig = -1.0e30f;
+constexpr float kNoMax = 16384.f;  // minus the "max" of a row without keys so far (log2 domain)
 
 __device__ inline float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ inline float shfl_xor_f(float x, int mask) { return __shfl_xor(x, mask, 64); }
@@ -233,15 +234,19 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_mfma_kernel(
 // ---------------------------------------------------------------------------
 // LDS-tiled MFMA prefill (bf16, D in {64, 128}).
 //
-// Workgroup = 16 / NT wavefronts sharing one kv head.  Keys are streamed in tiles
+// Workgroup = W wavefronts sharing one kv head.  Keys are streamed in tiles
 // of 64 (4 cache blocks).  Each tile of K and V is copied HBM -> LDS once per
-// workgroup with global_load_lds (no register staging) into one of three
-// LDS buffers, two tiles ahead of use, and read by all wavefronts.
-// Wavefront w owns 16 * NT query rows (NT MFMA column tiles) of one query
-// head; with group size G the workgroup covers min(G, 4) heads of the group
-// x (256 / min(G, 4)) query tokens, so every K/V byte brought into LDS feeds
-// 256 query rows.  NT = 2 keeps a wavefront within 256 registers, so two
-// wavefronts share each SIMD and one's softmax overlaps the other's MFMAs.
+// workgroup with global_load_lds (no register staging) into one of three or
+// four LDS buffers, two or three tiles ahead of use, and read by all
+// wavefronts.  A wavefront owns 16 * NT query rows (NT MFMA column tiles) of
+// one query head; with group size G the workgroup covers min(G, 4) heads of
+// the group.  KG = 1: every wavefront works on whole tiles, the workgroup on
+// 256 query rows (NT = 2, W = 8; a wavefront stays within 256 registers, so
+// two share each SIMD and one's softmax overlaps the other's MFMAs), so
+// every K/V byte brought into LDS feeds 256 rows.  KG = 2, for launches that
+// would leave CUs idle: half the wavefronts take the first 32 keys of each
+// tile and half the second, for 128 (NT = 2) or 64 (NT = 1) query rows, and
+// the two groups' results meet in LDS at the end.
 //
 // Per wavefront the 32-key steps form a software pipeline: the Sᵀ = K·Qᵀ
 // products of step n + 1 are issued in the same basic block as the
@@ -259,17 +264,13 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_mfma_kernel(
 //   V tile [4 blocks][D][16]: the two 16-byte halves of a 32-byte dim row d
 //     are swapped when bits 2 and 3 of d differ.
 //
-// Workgroup -> work mapping is XCD-aware: workgroups are dealt round-robin
-// to the 8 XCDs, so consecutive logical work items are remapped to the
-// same XCD; a logical chunk holds all query tiles of one kv head for all
-// sequences, and the tiles that share K/V then share that XCD's L2.  Within
-// a chunk the sequences go from most to least work, and within a sequence
-// the later (longer) query tiles go first.
-template <int D, int NT, typename TC>
-__global__ __launch_bounds__(64 * (16 / NT)) void prefill_tiled_kernel(
+// Sequences whose tiles a launch numbers through (see the work items below).
+constexpr int kMaxSeqs = 256;
+template <int D, int NT, int W, int KG, typename TC>
+__global__ __launch_bounds__(64 * W) void prefill_tiled_kernel(
     uint16_t* __restrict__ out, const uint16_t* __restrict__ q, const TC* __restrict__ kc,
     const TC* __restrict__ vc, const int32_t* __restrict__ block_tables, int mbs,
-    const int32_t* __restrict__ cu_q, const int32_t* __restrict__ past_lens, int Hq, int Hkv,
+    const int32_t* __restrict__ cu_q, const int32_t* __restrict__ past_lens, int Hq, int Hkv, int G,
     int num_blocks, float scale_log2, int B, int tiles_per_seq, int head_groups, int64_t q_row,
     int total_q, int max_q) {
   constexpr int KS = D / 32;   // QK reduction steps
@@ -280,8 +281,10 @@ __global__ __launch_bounds__(64 * (16 / NT)) void prefill_tiled_kernel(
   constexpr int ES = sizeof(TC);
   constexpr int CPR = D * ES / 16;  // 16-byte chunks per K row
   constexpr int KT = 64;       // keys per LDS tile
-  constexpr int W = 16 / NT;   // wavefronts per workgroup (64 query rows x 4 heads)
-  constexpr int NBUF = 3;      // LDS tile buffers
+  // LDS tile buffers, and how many tiles ahead of use a tile is copied.  KG =
+  // 2 has half the work per tile to cover a copy's latency.
+  constexpr int NBUF = KG == 2 && !FP8 ? 4 : 3;
+  constexpr int AHEAD = FP8 ? 3 : NBUF - 1;
   constexpr int TILE_BYTES = KT * D * ES;  // one K (or V) tile
   constexpr int NCH = TILE_BYTES / 1024;   // 1 KB copy chunks per tile
   constexpr int DMA_PER_WAVE = NCH >= W ? NCH / W : 1;
@@ -302,55 +305,130 @@ __global__ __launch_bounds__(64 * (16 / NT)) void prefill_tiled_kernel(
   const int lane = threadIdx.x & 63;
   const int wave_s = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
   const int c = lane & 15, j = lane >> 4;
-  const int G = Hq / Hkv;
-  const int HW = G < 4 ? G : 4;        // heads per workgroup
-  const int TT = 64 * (4 / HW);        // query tokens per workgroup
+  // G query heads per kv head, HW of them per workgroup, TT query tokens per
+  // workgroup (a power of two; quotients by runtime values are kept out of
+  // the way of a short launch, ~200 cycles each)
+  const int HW = G < 4 ? G : 4;
+  constexpr int TSH = NT * (W / KG / 4) == 4 ? 6 : NT * (W / KG / 4) == 2 ? 5 : 4;
+  static_assert(16 * NT * (W / KG / 4) == 1 << TSH, "query tokens per workgroup");
+  const int tsh = TSH + (HW == 1 ? 2 : HW == 2 ? 1 : 0), TT = 1 << tsh;
+  auto tiles_of = [&](int len) -> int { return (len + TT - 1) >> tsh; };
 
-  // Work items (logical ids): kv head (group) major, then sequences from the
-  // most to the least attention work (work = q_len * (past + q_len / 2),
-  // ties by index; past 64 sequences the index order), then query tiles
-  // longest first.  The items are cut into 8 contiguous chunks, one per XCD
-  // (workgroups are dealt round-robin to the XCDs, so workgroup g runs on XCD
-  // g % 8), and the items of one chunk stream the same kv head's K/V through
-  // that XCD's L2.  The grid is persistent (about one workgroup per CU): the
-  // XCD's workgroups take its chunk in rounds of nslot items, the workgroup
-  // in slot s taking item s of even rounds and item nslot - 1 - s of odd
-  // rounds (within a sequence the tiles go longest first, so this pairs long
-  // and short tiles); the workgroups stay on neighbouring items (the same
-  // sequence's K/V) and none waits for a CU behind a long-running one.
-  const int total = B * Hkv * head_groups * tiles_per_seq;
-  const int per_xcd = (total + 7) / 8;
-  const int xcd = (int)(blockIdx.x % 8), nslot = (int)(gridDim.x / 8), slot = (int)(blockIdx.x / 8);
-  const int lo = min(total, xcd * per_xcd), hi = min(total, lo + per_xcd);
-  __shared__ int seq_of_rank[64];
-  if (B <= 64 && (int)threadIdx.x < B) {
-    auto work = [&](int b) -> long long {
-      const QRange r = q_range(cu_q, past_lens, b, total_q, max_q);
-      return (long long)r.len * (2 * (long long)r.past + r.len);
-    };
-    const int b = threadIdx.x;
-    const long long wb = work(b);
-    int r = 0;
-    for (int o2 = 0; o2 < B; ++o2) {
-      const long long wo = work(o2);
-      r += (wo > wb) || (wo == wb && o2 < b);
+  // Work items: a query tile (TT tokens) of a sequence for one kv head
+  // (group).  Only tiles that hold query rows count: the sequences' tiles are
+  // numbered through, sequences with the most keys first and within one the
+  // later (longer) tiles first, by ranks and prefix sums that every workgroup
+  // forms in LDS (up to kMaxSeqs sequences; beyond, in index order with the
+  // empty tiles of the shorter sequences among them).
+  // The items of one kv head group go to one XCD (workgroups are dealt
+  // round-robin to the 8 XCDs, so workgroup g runs on XCD g % 8), whose L2
+  // then holds its K/V: with fewer groups than XCDs, a group's items are dealt
+  // in turn to its share of the XCDs.  The grid is persistent (about one
+  // workgroup per CU): the XCD's workgroups take its items in rounds of
+  // nslot, the workgroup in slot s taking item s of even rounds and item
+  // nslot - 1 - s of odd rounds (longest first, so this pairs long and short
+  // ones); the workgroups stay on neighbouring items (the same sequence's
+  // K/V) and none waits for a CU behind a long-running one.
+  // (Numbering max_q / TT tiles for every sequence instead, the single valid
+  // tiles of short sequences met the same few workgroups in every round: 29
+  // decode rows beside a 512-token chunk took 137 us; 32 prompts of 64 to 512
+  // tokens over 2 kv heads, where a group's two XCDs also got its longer and
+  // its shorter half, 47 us.)
+  __shared__ int rank_seq[kMaxSeqs], rank_begin[kMaxSeqs], rank_len[kMaxSeqs],
+      rank_past[kMaxSeqs], rank_tile0[kMaxSeqs], rank_of[kMaxSeqs], tile0_of[kMaxSeqs];
+  __shared__ int tiles_in_all;
+  const bool compact = B <= kMaxSeqs;
+  if (compact) {
+    // each wavefront compares its share of the sequences (held a lane each
+    // and read lane by lane) with all of them; the counts meet in LDS
+    for (int b = threadIdx.x; b < B; b += 64 * W) rank_of[b] = tile0_of[b] = 0;
+    __syncthreads();
+    for (int o0 = 0; o0 < B; o0 += 64) {
+      const QRange ro = q_range(cu_q, past_lens, min(o0 + lane, B - 1), total_q, max_q);
+      const int okey = ro.past + ro.len, otiles = tiles_of(ro.len), n = min(B - o0, 64);
+      for (int b0 = 0; b0 < B; b0 += 64) {
+        const int b = b0 + lane;
+        int key = okey;
+        if (b0 != o0) {
+          const QRange r = q_range(cu_q, past_lens, min(b, B - 1), total_q, max_q);
+          key = r.past + r.len;
+        }
+        int rank = 0, before = 0;
+        for (int i = wave_s; i < n; i += W) {
+          const int ko = __builtin_amdgcn_readlane(okey, i);
+          const bool first = ko > key || (ko == key && o0 + i < b);
+          rank += first;
+          before += first ? __builtin_amdgcn_readlane(otiles, i) : 0;
+        }
+        if (b < B && rank > 0) {
+          atomicAdd(&rank_of[b], rank);
+          atomicAdd(&tile0_of[b], before);
+        }
+      }
     }
-    seq_of_rank[r] = b;
+    __syncthreads();
+    for (int b = threadIdx.x; b < B; b += 64 * W) {
+      const QRange r = q_range(cu_q, past_lens, b, total_q, max_q);
+      const int rank = rank_of[b], before = tile0_of[b];
+      rank_seq[rank] = b;
+      rank_begin[rank] = r.begin;
+      rank_len[rank] = r.len;
+      rank_past[rank] = r.past;
+      rank_tile0[rank] = before;
+      if (rank == B - 1) tiles_in_all = before + tiles_of(r.len);
+    }
+    __syncthreads();
   }
-  __syncthreads();
-  auto seq_of = [&](int rank) -> int { return B <= 64 ? seq_of_rank[rank] : rank; };
+  const int nq = compact ? tiles_in_all : B * tiles_per_seq;  // tiles per kv head group
+  const int nkg = Hkv * head_groups;
+  const int xcd = (int)(blockIdx.x % 8), nslot = (int)(gridDim.x / 8), slot = (int)(blockIdx.x / 8);
+  // the XCD's items: item i is tile (t0 + i * dt) % nq of group g0 + (t0 + i * dt) / nq
+  // (the quotient is 0 where the XCD has one group)
+  int g0 = 0, t0 = 0, dt = 1, items;
+  if (nkg == 1 || nkg == 2 || nkg == 4 || nkg == 8) {
+    const int sh = nkg == 1 ? 3 : nkg == 2 ? 2 : nkg == 4 ? 1 : 0;
+    dt = 1 << sh;
+    g0 = xcd >> sh;
+    t0 = xcd & (dt - 1);
+    items = t0 < nq ? (nq - t0 + dt - 1) >> sh : 0;
+  } else {
+    const int total = nkg * nq, per_xcd = (total + 7) / 8;
+    t0 = min(total, xcd * per_xcd);
+    items = min(total, t0 + per_xcd) - t0;
+  }
 
   // One work item: attention for one (kv head group, sequence, query tile).
-  auto process = [&](int logical) {
+  auto process = [&](int item) {
+  int kvhg = g0, qt = t0 + item * dt;
+  if (qt >= nq) {
+    kvhg += qt / nq;
+    qt %= nq;
+  }
   // every wavefront is done with the previous item's LDS tiles
   __syncthreads();
-  const int kvhg = logical / (B * tiles_per_seq);
-  const int rem = logical % (B * tiles_per_seq);
-  const int tile = tiles_per_seq - 1 - rem % tiles_per_seq;
-  const int seq = seq_of(rem / tiles_per_seq);
-  const int kvh = kvhg / head_groups, hg = kvhg % head_groups;
-
-  const QRange qr = q_range(cu_q, past_lens, seq, total_q, max_q);
+  int seq, tile;
+  QRange qr;
+  if (compact) {
+    // the last rank whose tiles begin at or before this one
+    int r = -1;
+    for (int b0 = 0; b0 < B; b0 += 64)
+      r += __builtin_popcountll(__builtin_amdgcn_ballot_w64(
+          b0 + lane < B && rank_tile0[min(b0 + lane, B - 1)] <= qt));
+    seq = __builtin_amdgcn_readfirstlane(rank_seq[r]);
+    qr.begin = __builtin_amdgcn_readfirstlane(rank_begin[r]);
+    qr.len = __builtin_amdgcn_readfirstlane(rank_len[r]);
+    qr.past = __builtin_amdgcn_readfirstlane(rank_past[r]);
+    tile = tiles_of(qr.len) - 1 - (qt - __builtin_amdgcn_readfirstlane(rank_tile0[r]));
+  } else {
+    seq = qt / tiles_per_seq;
+    tile = tiles_per_seq - 1 - qt % tiles_per_seq;
+    qr = q_range(cu_q, past_lens, seq, total_q, max_q);
+  }
+  int kvh = kvhg, hg = 0;
+  if (head_groups > 1) {
+    kvh = kvhg / head_groups;
+    hg = kvhg % head_groups;
+  }
   const int q_begin = qr.begin;
   const int qlen = qr.len;
   const int tok0 = tile * TT;
@@ -360,36 +438,15 @@ __global__ __launch_bounds__(64 * (16 / NT)) void prefill_tiled_kernel(
   const int n_kt = (key_end + KT - 1) / KT;
   const int nblk = (key_end + kBlock - 1) / kBlock;
 
-  const int hl = wave_s % HW, tsub = wave_s / HW;
+  // KG = 2: wavefronts W/2 .. take the second 32 keys of every tile
+  const int kgrp = KG == 2 ? wave_s / (W / 2) : 0, wt = KG == 2 ? wave_s % (W / 2) : wave_s;
+  const int tsub = (wt * (HW == 4 ? 8 : HW == 3 ? 11 : HW == 2 ? 16 : 32)) >> 5;  // wt / HW
+  const int hl = wt - tsub * HW;
   const int head_in_group = hg * 4 + hl;
-  const bool wave_active = wave_s < HW * (TT / (16 * NT)) && head_in_group < G;
+  const bool wave_active = tsub < (TT / (16 * NT)) && head_in_group < G;
   const int head = kvh * G + head_in_group;
   const int r0 = tok0 + tsub * 16 * NT;  // first query row of this wavefront
   const bool rows_active = wave_active && r0 < qlen;
-
-  bf16x8 qv[NT][KS];
-  f32x4 o[NT][DT];
-  f32x4 lacc[NT];  // softmax denominators, accumulated on the matrix core
-  float nm[NT];  // minus the rows' running maxima (the Sᵀ accumulators start at it)
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    const int row = r0 + 16 * nt + c;
-#pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      if (rows_active && row < qlen) {
-        const bf16x8 raw = *reinterpret_cast<const bf16x8*>(
-            q + (int64_t)(q_begin + row) * q_row + (int64_t)head * D + 32 * s + 8 * j);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) qv[nt][s][i] = (__bf16)((float)raw[i] * scale_log2);
-      } else {
-        qv[nt][s] = bf16x8{};
-      }
-    }
-    nm[nt] = 0.f;
-    lacc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) o[nt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
 
   // Block ids.  Each wavefront's HBM -> LDS copies of a tile all read one
   // cache block (block `wblk` of the tile's 4), so a wavefront needs just
@@ -405,12 +462,6 @@ __global__ __launch_bounds__(64 * (16 / NT)) void prefill_tiled_kernel(
   const int32_t* btab = block_tables + (int64_t)seq * mbs;
   const int64_t head_stride = (int64_t)kBlock * D;
   const int wblk = (wave_s * DMA_PER_WAVE) / CPB;
-  int bad = 0;
-  for (int b = threadIdx.x; b < nblk; b += blockDim.x) {
-    const int32_t id = btab[b];
-    bad |= (id < 0 || id >= num_blocks) ? 1 : 0;
-  }
-  const bool bad_ids = __syncthreads_or(bad) != 0;
   auto load_ids = [&](int base) -> int32_t {
     const int t = base + lane;
     if (t >= n_kt) return 0;
@@ -419,6 +470,24 @@ __global__ __launch_bounds__(64 * (16 / NT)) void prefill_tiled_kernel(
   };
   int ids_base = 0;
   int32_t ids = load_ids(0);
+  // The query rows (clamped: unconditional loads, all in flight together
+  // with the ids; converted after the first tiles' copies are issued) and
+  // the check of the table's ids.
+  bf16x8 qv[NT][KS];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    const int row = min(r0 + 16 * nt + c, qlen - 1);
+    const uint16_t* qp = q + (int64_t)(q_begin + row) * q_row +
+                         (int64_t)(kvh * G + min(head_in_group, G - 1)) * D + 8 * j;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) qv[nt][s] = *reinterpret_cast<const bf16x8*>(qp + 32 * s);
+  }
+  int bad = 0;
+  for (int b = threadIdx.x; b < nblk; b += 64 * W) {
+    const int32_t id = btab[b];
+    bad |= (id < 0 || id >= num_blocks) ? 1 : 0;
+  }
+  bool bad_ids = false;  // set after the first copies are issued
   auto fetch_id = [&](int kt) -> int32_t {
     if (kt - ids_base >= 64) {  // wavefront-uniform
       ids_base = kt & ~63;
@@ -494,6 +563,18 @@ __global__ __launch_bounds__(64 * (16 / NT)) void prefill_tiled_kernel(
           16, 0, 0);
     }
   };
+  // Waits until at most `n` (0 to 2) tiles' copies of this wavefront are in
+  // flight.
+  auto wait_tiles = [&](int n) __attribute__((always_inline)) {
+    constexpr int P = 2 * DMA_PER_WAVE;
+    static_assert(2 * P < 64, "vmcnt");
+    if (n >= 2)
+      __builtin_amdgcn_s_waitcnt(0x0F70 | ((2 * P) & 0xF) | (((2 * P) >> 4) << 14));
+    else if (n == 1)
+      __builtin_amdgcn_s_waitcnt(0x0F70 | (P & 0xF) | ((P >> 4) << 14));
+    else
+      __builtin_amdgcn_s_waitcnt(0x0F70);
+  };
   // A tile that reaches past the last key, or holds a block id outside the
   // pool, has V entries that are not this sequence's data (any bits, NaN
   // included).  Zero them in LDS once, after the tile has landed, so P·V
@@ -503,14 +584,24 @@ __global__ __launch_bounds__(64 * (16 / NT)) void prefill_tiled_kernel(
   auto zero_stale = [&](int kt, int buf, int valid) -> bool {
     const bool special = kt * KT + KT > key_end || valid != (1 << (KT / kBlock)) - 1;
     if (!special) return false;
-    uint16_t* vz = reinterpret_cast<uint16_t*>(&smem[1][buf][0]);
-    for (int e = threadIdx.x; e < KT * D; e += blockDim.x) {
-      const int key = e / D, d = e % D;
-      const int b = key / kBlock, t16 = key % kBlock;
-      const bool ok = kt * KT + key < key_end && ((valid >> b) & 1);
-      if (!ok) {
-        const int half = (t16 / 8) ^ vswz(d);
-        vz[(b * D + d) * kBlock + half * 8 + t16 % 8] = 0;
+    // one 32-byte dim row (16 keys of a block) per thread, in 16-byte halves
+    for (int e = threadIdx.x; e < KT / kBlock * D; e += 64 * W) {
+      const int b = e / D, d = e % D;
+      const int lim = (valid >> b) & 1 ? key_end - kt * KT - b * kBlock : 0;  // keys to keep
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int n = lim - 8 * h;
+        if (n >= 8) continue;
+        uint4* half = reinterpret_cast<uint4*>(&smem[1][buf][e * 32 + (h ^ vswz(d)) * 16]);
+        uint4 v = uint4{0, 0, 0, 0};
+        if (n > 0) {
+          v = *half;
+          uint32_t* w = &v.x;
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            w[i] = n >= 2 * i + 2 ? w[i] : n == 2 * i + 1 ? w[i] & 0xFFFFu : 0u;
+        }
+        *half = v;
       }
     }
     __syncthreads();
@@ -569,8 +660,7 @@ __global__ __launch_bounds__(64 * (16 / NT)) void prefill_tiled_kernel(
   // kk's row i holds key 8 (i / 4) + 4 kk + i % 4 of the step, so the lane
   // (c, j) that receives rows 4j .. 4j+3 of both tiles holds keys
   // 8j .. 8j+7: eight consecutive keys of block j / 2.
-  auto qk_load = [&](int buf, auto stc, bf16x8 (&ka)[2][KS]) {
-    constexpr int ST = decltype(stc)::value;
+  auto qk_load = [&](int buf, int ST, bf16x8 (&ka)[2][KS]) __attribute__((always_inline)) {
     const uint8_t* ks = &smem[0][buf][0];
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
@@ -597,23 +687,39 @@ __global__ __launch_bounds__(64 * (16 / NT)) void prefill_tiled_kernel(
 
   bool tile_special;        // current tile needs key masking
   int valid_cur;            // validity bits of the current tile's 4 blocks
-  int32_t id_ahead = 0;     // this wavefront's block id of the tile two (FP8: three) ahead
+  int32_t id_ahead = 0;     // this wavefront's block id of the tile AHEAD of this one
   // Prologue: tiles 0 and 1 in flight, wait for tile 0.  (FP8: tiles 0 and
   // 1 staged and converted, then tile 2 copied into slot 0.)
   issue_tile(fetch_id(0), 0);
+  if (n_kt > 1) issue_tile(fetch_id(1), 1);
+  if constexpr (AHEAD == 3 && !FP8)
+    if (n_kt > 2) issue_tile(fetch_id(2), 2);
+  f32x4 o[NT][DT];
+  f32x4 lacc[NT];  // softmax denominators, accumulated on the matrix core
+  float nm[NT];  // minus the rows' running maxima (the Sᵀ accumulators start at it)
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    const bool ok = rows_active && r0 + 16 * nt + c < qlen;
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        qv[nt][s][i] = (__bf16)(ok ? (float)qv[nt][s][i] * scale_log2 : 0.f);
+    nm[nt] = 0.f;
+    lacc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) o[nt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  bad_ids = __syncthreads_or(bad) != 0;
   if constexpr (FP8) {
-    if (n_kt > 1) issue_tile(fetch_id(1), 1);
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    wait_tiles(0);
     __syncthreads();
     convert_tile(0, 0);
     if (n_kt > 1) convert_tile(1, 1);
     __syncthreads();
     if (n_kt > 2) issue_tile(fetch_id(2), 0);
-  } else if (n_kt > 1) {
-    issue_tile(fetch_id(1), 1);
-    __builtin_amdgcn_s_waitcnt(0x0F70 | ((2 * DMA_PER_WAVE) & 0xF) | (((2 * DMA_PER_WAVE) >> 4) << 14));
   } else {
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    wait_tiles(min(n_kt, AHEAD) - 1);
   }
   __syncthreads();
   valid_cur = tile_valid(0);
@@ -625,7 +731,7 @@ __global__ __launch_bounds__(64 * (16 / NT)) void prefill_tiled_kernel(
   f32x4 S0[NT][2], S1[NT][2];
   {
     bf16x8 ka[2][KS];
-    qk_load(0, IC<0>{}, ka);
+    qk_load(0, kgrp, ka);
     qk_mfma(ka, S0);
   }
 
@@ -633,9 +739,13 @@ __global__ __launch_bounds__(64 * (16 / NT)) void prefill_tiled_kernel(
   // softmax of S (already computed), then in one basic block the P·V
   // products of this step and the Sᵀ products of the next.
   auto step = [&](int buf, auto stc, int kt, f32x4 (&S)[NT][2], f32x4 (&Snext)[NT][2]) {
-    constexpr int ST = decltype(stc)::value;
+    // KG = 1: step STC of the tile; KG = 2: this group's one step of it, which
+    // begins with the tile boundary as the second step does
+    constexpr int STC = KG == 2 ? 1 : decltype(stc)::value;
+    const int ST = KG == 2 ? kgrp : STC;
     const int next = buf == NBUF - 1 ? 0 : buf + 1;
-    const int ahead = next == NBUF - 1 ? 0 : next + 1;
+    // the buffer of the tile before this one, free again at the boundary
+    const int free_buf = buf == 0 ? NBUF - 1 : buf - 1;
     // This step's Vᵀ fragments (dims 16 dt + c, keys 8j .. 8j+7 = one
     // 16-byte half of the 32-byte row of block 2 ST + j / 2), read first so
     // the softmax covers their latency.
@@ -651,19 +761,23 @@ __global__ __launch_bounds__(64 * (16 / NT)) void prefill_tiled_kernel(
     // K fragments of the next step, read now so the softmax prep below
     // covers their LDS latency.
     bf16x8 ka[2][KS];
-    if constexpr (ST == 0) {
-      qk_load(buf, IC<1>{}, ka);
+    if constexpr (KG == 2) {
+      if (kt + AHEAD < n_kt) id_ahead = fetch_id(kt + AHEAD);
+    }
+    if constexpr (STC == 0) {
+      qk_load(buf, 1, ka);
       // this wavefront's block of the tile two ahead, a step before its copy
-      if (kt + (FP8 ? 3 : 2) < n_kt) id_ahead = fetch_id(kt + (FP8 ? 3 : 2));
+      if (kt + AHEAD < n_kt) id_ahead = fetch_id(kt + AHEAD);
     } else {
       // Tile boundary, at the start of a tile's second step: the next tile
-      // has landed (all waves), the buffer two tiles ahead is free again
+      // has landed (all waves), the previous tile's buffer is free again
       // (every wavefront has finished the tile before this one), and the
       // next tile's first K fragments are read now so this step's softmax
       // covers them.  Past the last tile they are read from a buffer of
       // stale data and the products are never used.
       if (kt + 1 < n_kt) {
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): only tile kt + 1 is in flight
+        // tile kt + 1 has landed; with four buffers kt + 2 may be in flight
+        wait_tiles(NBUF == 4 && kt + 2 < n_kt ? 1 : 0);
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
@@ -672,13 +786,13 @@ __global__ __launch_bounds__(64 * (16 / NT)) void prefill_tiled_kernel(
           // compute buffer, visible to all at the next boundary's barrier;
           // its staging slot's previous tile (kt + 1) was converted a tile
           // ago, so tile kt + 3 is copied into it
-          if (kt + 2 < n_kt) convert_tile(ahead, (kt + 2) & 1);
+          if (kt + 2 < n_kt) convert_tile(free_buf, (kt + 2) & 1);
           if (kt + 3 < n_kt) issue_tile(id_ahead, (kt + 3) & 1);
         } else {
-          if (kt + 2 < n_kt) issue_tile(id_ahead, ahead);
+          if (kt + AHEAD < n_kt) issue_tile(id_ahead, free_buf);
         }
       }
-      qk_load(next, IC<0>{}, ka);
+      qk_load(next, kgrp, ka);
     }
     {
       const int kb = (2 * kt + ST) * 32;  // first key of this step; x[i] <-> key kb + 8j + i
@@ -710,15 +824,16 @@ __global__ __launch_bounds__(64 * (16 / NT)) void prefill_tiled_kernel(
       // only then is the exact max formed across the four lanes of the row
       // and the accumulator rescaled.  The first step always sets the max
       // (m starts at 0, which says nothing about the row's scores).
-      const bool first = ST == 0 && kt == 0;
+      const bool first = (KG == 2 || STC == 0) && kt == 0;
       if (first || __builtin_amdgcn_ballot_w64(need)) {
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
           float bm = lm[nt];
           bm = fmaxf(bm, shfl_xor_f(bm, 16));
           bm = fmaxf(bm, shfl_xor_f(bm, 32));
-          // a row with every key of the first step masked keeps m = 0
-          const float delta = first ? (bm > -INFINITY ? bm : 0.f) : fmaxf(bm, 0.f);
+          // a row with every key of the first step masked starts from a max
+          // so low that its first key exceeds it
+          const float delta = first ? (bm > -INFINITY ? bm : -kNoMax) : fmaxf(bm, 0.f);
           nm[nt] -= delta;
 #pragma unroll
           for (int i = 0; i < 8; ++i) S[nt][i >> 2][i & 3] -= delta;
@@ -788,7 +903,7 @@ __global__ __launch_bounds__(64 * (16 / NT)) void prefill_tiled_kernel(
       for (int nt = 0; nt < NT; ++nt)
         lacc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pb[nt], lacc[nt], 0, 0, 0);
     }
-    if constexpr (ST == 1) {
+    if constexpr (STC == 1) {
       if (kt + 1 < n_kt) {
         valid_cur = tile_valid(kt + 1);
         tile_special = zero_stale(kt + 1, next, valid_cur);
@@ -800,8 +915,50 @@ __global__ __launch_bounds__(64 * (16 / NT)) void prefill_tiled_kernel(
   // buffers, which would make every LDS address an immediate offset, costs
   // register spills.)
   for (int kt = 0, buf = 0; kt < n_kt; ++kt, buf = buf == NBUF - 1 ? 0 : buf + 1) {
-    step(buf, IC<0>{}, kt, S0, S1);
-    step(buf, IC<1>{}, kt, S1, S0);
+    if constexpr (KG == 2) {
+      step(buf, IC<1>{}, kt, S0, S1);
+      if (++kt == n_kt) break;
+      buf = buf == NBUF - 1 ? 0 : buf + 1;
+      step(buf, IC<1>{}, kt, S1, S0);
+    } else {
+      step(buf, IC<0>{}, kt, S0, S1);
+      step(buf, IC<1>{}, kt, S1, S0);
+    }
+  }
+
+  if constexpr (KG == 2) {
+    // The two groups' results meet in LDS (the tiles' space): log-sum-exp
+    // merge by the first group's wavefronts.  A group that saw no key of a
+    // row (l = 0) drops out.
+    static_assert(W / 2 * NT * (DT * 1024 + 512) <= 2 * NBUF * CT_BYTES, "merge space");
+    float* mo = reinterpret_cast<float*>(&smem[0][0][0]);
+    float* mml = mo + W / 2 * NT * DT * 256;
+    __syncthreads();
+    if (kgrp == 1) {
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) {
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+          *reinterpret_cast<f32x4*>(mo + ((wt * NT + nt) * DT + dt) * 256 + lane * 4) = o[nt][dt];
+        *reinterpret_cast<float2*>(mml + ((wt * NT + nt) * 64 + lane) * 2) =
+            float2{-nm[nt], lacc[nt][0]};
+      }
+    }
+    __syncthreads();
+    if (kgrp == 1) return;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      const float2 ml = *reinterpret_cast<const float2*>(mml + ((wt * NT + nt) * 64 + lane) * 2);
+      const float ma = lacc[nt][0] != 0.f ? -nm[nt] : kNegBig;
+      const float mb = ml.y != 0.f ? ml.x : kNegBig;
+      const float mx = fmaxf(ma, mb);
+      const float fa = fast_exp2(ma - mx), fb = fast_exp2(mb - mx);
+      lacc[nt] = lacc[nt] * fa + ml.y * fb;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+        o[nt][dt] = o[nt][dt] * fa +
+                    *reinterpret_cast<const f32x4*>(mo + ((wt * NT + nt) * DT + dt) * 256 + lane * 4) * fb;
+    }
   }
 
   if (!rows_active) return;
@@ -816,14 +973,14 @@ __global__ __launch_bounds__(64 * (16 / NT)) void prefill_tiled_kernel(
     for (int dt = 0; dt < DT; ++dt) {
       uint16_t w[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) w[r] = f32_to_bf16_bits(o[nt][dt][r] * inv);
+      for (int r = 0; r < 4; ++r) w[r] = __builtin_bit_cast(uint16_t, (__bf16)(o[nt][dt][r] * inv));
       *reinterpret_cast<uint64_t*>(orow + 16 * dt) = *reinterpret_cast<const uint64_t*>(w);
     }
   }
   };
-  for (int r = 0; lo + r * nslot < hi; ++r) {
-    const int item = lo + r * nslot + ((r & 1) ? nslot - 1 - slot : slot);
-    if (item < hi) process(item);
+  for (int r = 0; r * nslot < items; ++r) {
+    const int item = r * nslot + ((r & 1) ? nslot - 1 - slot : slot);
+    if (item < items) process(item);
   }
 }
 
@@ -955,34 +1112,52 @@ int32_t prefill_impl(void* out, const void* q, const void* k_cache, const void* 
   if (tiled) {
     const int G = num_heads / num_kv_heads;
     const int HW = G < 4 ? G : 4;
-    const int TT = 64 * (4 / HW);
-    const int tiles_per_seq = (max_q_len + TT - 1) / TT;
     const int head_groups = (G + 3) / 4;
-    const long long total = (long long)num_seqs * num_kv_heads * head_groups * tiles_per_seq;
-    PA_REQUIRE(total < (1ll << 31) / 8, PA_ERR_UNSUPPORTED, "pa_prefill: launch too large");
-    const int per_xcd = (int)((total + 7) / 8);
-    // persistent grid: about one workgroup per CU (a multiple of the 8 XCDs)
-    const dim3 grid(8 * std::max(1, std::min(per_xcd, compute_units() / 8)));
     auto* o = (uint16_t*)out;
     auto* qq = (const uint16_t*)q;
-    constexpr int NT = 2;
-#define PA_LAUNCH_TILED(DD, TC)                                                               \
-  prefill_tiled_kernel<DD, NT, TC><<<grid, 64 * (16 / NT), 0, s>>>(                           \
-      o, qq, (const TC*)k_cache, (const TC*)v_cache, block_tables, max_blocks_per_seq,        \
-      cu_q_lens, past_lens, num_heads, num_kv_heads, num_blocks, scale_log2, num_seqs,        \
-      tiles_per_seq, head_groups, q_row, total_q, max_q_len)
-    if (fp8) {
-      if (head_dim == 128)
-        PA_LAUNCH_TILED(128, uint8_t);
-      else
-        PA_LAUNCH_TILED(64, uint8_t);
-    } else {
-      if (head_dim == 128)
-        PA_LAUNCH_TILED(128, uint16_t);
-      else
-        PA_LAUNCH_TILED(64, uint16_t);
-    }
-#undef PA_LAUNCH_TILED
+    auto launch = [&](auto dc, auto ntc, auto wc, auto kgc, auto cache) -> int32_t {
+      constexpr int DD = decltype(dc)::value, NT = decltype(ntc)::value, W = decltype(wc)::value;
+      constexpr int KG = decltype(kgc)::value;
+      using TC = decltype(cache);
+      const int TT = 16 * NT * (W / KG / 4) * (4 / HW);
+      const int tiles_per_seq = (max_q_len + TT - 1) / TT;
+      const long long total = (long long)num_seqs * num_kv_heads * head_groups * tiles_per_seq;
+      PA_REQUIRE(total < (1ll << 31) / 8, PA_ERR_UNSUPPORTED, "pa_prefill: launch too large");
+      const int per_xcd = (int)((total + 7) / 8);
+      // persistent grid: about one workgroup per CU (a multiple of the 8 XCDs)
+      const dim3 grid(8 * std::max(1, std::min(per_xcd, compute_units() / 8)));
+      prefill_tiled_kernel<DD, NT, W, KG, TC><<<grid, 64 * W, 0, s>>>(
+          o, qq, (const TC*)k_cache, (const TC*)v_cache, block_tables, max_blocks_per_seq,
+          cu_q_lens, past_lens, num_heads, num_kv_heads, G, num_blocks, scale_log2, num_seqs,
+          tiles_per_seq, head_groups, q_row, total_q, max_q_len);
+      return PA_OK;
+    };
+    // Query tokens per workgroup.  An item's time is its keys times the
+    // workgroup's time per key tile (1 for 256 query rows, 0.7 for 128 rows
+    // with two key groups, 0.53 for 64), and the items of a launch share the
+    // CUs, their average about 0.65 of the longest; the lengths are on the
+    // device, so the items are counted from the totals.  Measured, us (256 /
+    // 128 / 64 rows): 512 tokens on 1024 cached, 32 / 8 heads x 128: 46 / 35
+    // / 26; 701, 123 and 411 on 3001, 0 and 517: 98 / 71 / 87 (FP8 115 / 85 /
+    // 119); 2 x 1024 on 0 and 1024: 61 / 54 / 71; 2048 on 2000 and 1000 on
+    // 0: 115 / 136 / 181; 4 x 2048: 260 / 307 / 427; 14 / 2 heads x 64: 500,
+    // 300, 222: 22 / 17 / 14, 2000, 1300, 1222: 45 / 55 / 75.
+    auto cost = [&](int tokens, double per_tile) -> double {
+      tokens *= HW == 1 ? 4 : HW == 2 ? 2 : 1;
+      const double tiles =
+          std::max((double)num_seqs, (double)total_q / tokens + 0.5 * num_seqs);
+      return per_tile * std::max(1., 0.65 / 256 * tiles * num_kv_heads * head_groups);
+    };
+    const double c64 = cost(64, 1.), c32 = cost(32, 0.7), c16 = cost(16, 0.53);
+    auto pick = [&](auto dc, auto cache) -> int32_t {
+      if (c64 <= c32 && c64 <= c16) return launch(dc, IC<2>{}, IC<8>{}, IC<1>{}, cache);
+      if (c32 <= c16) return launch(dc, IC<2>{}, IC<8>{}, IC<2>{}, cache);
+      return launch(dc, IC<1>{}, IC<8>{}, IC<2>{}, cache);
+    };
+    const int32_t rc = fp8 ? (head_dim == 128 ? pick(IC<128>{}, uint8_t{}) : pick(IC<64>{}, uint8_t{}))
+                           : (head_dim == 128 ? pick(IC<128>{}, uint16_t{})
+                                              : pick(IC<64>{}, uint16_t{}));
+    if (rc != PA_OK) return rc;
   } else if (mfma) {
     constexpr int NT = 2;
     const int rows_per_wg = 16 * NT * kWaves;
