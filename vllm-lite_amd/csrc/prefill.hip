@@ -13,6 +13,8 @@
 //    softmax per query row; the causal mask is only evaluated on steps that
 //    straddle the diagonal.  Four wavefronts per workgroup cover adjacent
 //    row ranges of the same head so their K/V reads share the L1/L2.
+//  * prefill_f32_kernel (f32, D in {16 .. 256}): the same products on the f32
+//    MFMA, with the keys split over wavefronts.
 //  * prefill_generic_kernel (f32 or bf16, any D <= 512): one wavefront per
 //    (query row, head), reference-grade.
 #include <algorithm>
@@ -984,6 +986,214 @@ __global__ __launch_bounds__(64 * W) void prefill_tiled_kernel(
   }
 }
 
+// f32 caches (plain, or int8-in-f32 with one scale per block), D in {16, 32,
+// 64, 128, 256}, on v_mfma_f32_16x16x4_f32 (full f32 products and sums).
+//
+// Workgroup = 8 wavefronts on 16 query tokens: min(G, 4) heads of one kv head
+// x 8 / that many key splits; a wavefront takes every KS-th step (NB blocks of
+// 16 keys) for the 16 tokens of its head, and the splits' results meet in LDS.
+// Operand lane layout (lane = 16 j + c; the MFMA contracts over j):
+//   Sᵀ = K·Qᵀ: a lane loads 4 consecutive dims 16 t + 4 j .. of key row c and
+//     query row c (16 bytes each) and feeds them to 4 MFMAs -> the lane holds
+//     Sᵀ[key 4 j + r][query c];
+//   Oᵀ = Vᵀ·Pᵀ: a lane loads keys 4 j .. 4 j + 3 of dim 16 dt + c (16 bytes of
+//     the token-minor block), whose P it already holds.
+// K and V go straight from the cache to operand registers; the heads of a
+// workgroup read the same blocks at the same time through the L1.
+// Bound: the f32 matrix rate (157 TFLOP/s) where there are enough tokens, else
+// the serial steps of the longest row tile, which the key splits shorten.
+// 511, 129, 300 and 64 tokens on 0, 256, 0 and 33, 14 / 2 heads x 64:
+// 492 us a call with one wavefront per (row, head) on the VALU, 27.7 here.
+template <int D>
+__global__ __launch_bounds__(512) void prefill_f32_kernel(
+    float* __restrict__ out, const float* __restrict__ q, const float* __restrict__ kc,
+    const float* __restrict__ vc, const int32_t* __restrict__ block_tables, int mbs,
+    const int32_t* __restrict__ cu_q, const int32_t* __restrict__ past_lens, int Hq, int Hkv, int G,
+    int num_blocks, float scale_log2, const float* __restrict__ kv_scales, int64_t q_row,
+    int total_q, int max_q) {
+  constexpr int NB = D <= 64 ? 2 : 1;  // cache blocks per step
+  constexpr int DT = D / 16;
+  __shared__ __attribute__((aligned(16))) float mo[8][DT][64][4];
+  __shared__ float mml[8][64][2];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 15, j = lane >> 4;
+  const int seq = blockIdx.z, head_groups = (G + 3) / 4;
+  const QRange qr = q_range(cu_q, past_lens, seq, total_q, max_q);
+  const int tok0 = 16 * (int)(gridDim.x - 1 - blockIdx.x);  // the longest tiles first
+  if (tok0 >= qr.len) return;
+  const int HW = min(G, 4), KS = HW == 1 ? 8 : HW == 2 ? 4 : 2;
+  const int ks = wave / HW, hl = wave - ks * HW;
+  const int kvh = blockIdx.y / head_groups, hig = (blockIdx.y - kvh * head_groups) * 4 + hl;
+  const bool active = ks < KS && hig < G;  // HW = 3 leaves two wavefronts, G % 4 heads over
+  const int head = kvh * G + min(hig, G - 1);
+  const int row_pos = qr.past + tok0 + c;  // this lane's query row
+  const int key_end = min(qr.past + min(qr.len, tok0 + 16), mbs * kBlock);
+  const int nblk = active ? (key_end + kBlock - 1) / kBlock : 0;
+
+  float4 qv[DT];
+  const float* qp = q + (int64_t)(qr.begin + min(tok0 + c, qr.len - 1)) * q_row +
+                    (int64_t)head * D + 4 * j;
+#pragma unroll
+  for (int t = 0; t < DT; ++t) qv[t] = *reinterpret_cast<const float4*>(qp + 16 * t);
+  f32x4 o[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = kNegBig, l = 0.f;
+  const int32_t* btab = block_tables + (int64_t)seq * mbs;
+  const int64_t head_stride = (int64_t)kBlock * D;
+
+  for (int ib = NB * ks; ib < nblk; ib += NB * KS) {
+    const float* vb[NB];
+    int lim[NB];  // keys of the block that count
+    float bscale[NB];
+    float4 kx[NB][DT], vx[NB][DT];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      int32_t id = btab[min(ib + b, nblk - 1)];
+      lim[b] = min(max(key_end - (ib + b) * kBlock, 0), kBlock);
+      if (id < 0 || id >= num_blocks) {
+        id = 0;
+        lim[b] = 0;
+      }
+      const int64_t off = ((int64_t)id * Hkv + kvh) * head_stride;
+      vb[b] = vc + off;
+      const float* kp = kc + off + c * D + 4 * j;
+#pragma unroll
+      for (int t = 0; t < DT; ++t) kx[b][t] = *reinterpret_cast<const float4*>(kp + 16 * t);
+      bscale[b] = kv_scales ? kv_scales[id] : 1.0f;
+    }
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+        vx[b][dt] = *reinterpret_cast<const float4*>(vb[b] + (16 * dt + c) * kBlock + 4 * j);
+    f32x4 S[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) S[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        S[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kx[b][t].x, qv[t].x, S[b], 0, 0, 0);
+        S[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kx[b][t].y, qv[t].y, S[b], 0, 0, 0);
+        S[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kx[b][t].z, qv[t].z, S[b], 0, 0, 0);
+        S[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kx[b][t].w, qv[t].w, S[b], 0, 0, 0);
+      }
+    // keys past the end, in invalid blocks or above a row's diagonal
+    const bool diag = (ib + NB) * kBlock - 1 > qr.past + tok0;  // wavefront-uniform
+    bool partial = false;
+    float x[NB][4], bm = -INFINITY;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      partial |= lim[b] < kBlock;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        x[b][r] = S[b][r] * (bscale[b] * scale_log2);
+        const int t = 4 * j + r;
+        if (t >= lim[b] || (ib + b) * kBlock + t > row_pos) x[b][r] = -INFINITY;
+        bm = fmaxf(bm, x[b][r]);
+      }
+    }
+    // the max is kept until a score exceeds it by 2^8 (see decode)
+    if (__builtin_amdgcn_ballot_w64(bm > m + 8.0f)) {
+      bm = fmaxf(bm, shfl_xor_f(bm, 16));
+      bm = fmaxf(bm, shfl_xor_f(bm, 32));
+      const float mn = fmaxf(m, bm);
+      const float a = exp2f(m - mn);
+      m = mn;
+      l *= a;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) o[dt] *= a;
+    }
+    float p[NB][4];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        p[b][r] = exp2f(x[b][r] - m);
+        l += p[b][r];
+        p[b][r] *= bscale[b];
+      }
+    if (partial) {
+      // cache contents past the context may be any bits
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+          const int n = lim[b] - 4 * j;
+          vx[b][dt] = float4{n > 0 ? vx[b][dt].x : 0.f, n > 1 ? vx[b][dt].y : 0.f,
+                             n > 2 ? vx[b][dt].z : 0.f, n > 3 ? vx[b][dt].w : 0.f};
+        }
+    }
+    if (diag) {
+      // A value that is not finite above a row's diagonal must not reach it
+      // through 0 * v: such a step goes key by key.
+      float odd = 0.f;
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+          odd += (vx[b][dt].x - vx[b][dt].x) + (vx[b][dt].y - vx[b][dt].y) +
+                 (vx[b][dt].z - vx[b][dt].z) + (vx[b][dt].w - vx[b][dt].w);
+      if (__builtin_amdgcn_ballot_w64(odd != 0.f)) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            for (int jj = 0; jj < 4; ++jj) {
+              const float pk = __shfl(p[b][r], 16 * jj + c, 64);
+              const int t = 4 * jj + r;
+              if (t >= lim[b] || (ib + b) * kBlock + t > row_pos) continue;
+#pragma unroll
+              for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                  o[dt][e] += pk * vb[b][(16 * dt + 4 * j + e) * kBlock + t];
+            }
+        continue;
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(vx[b][dt].x, p[b][0], o[dt], 0, 0, 0);
+        o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(vx[b][dt].y, p[b][1], o[dt], 0, 0, 0);
+        o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(vx[b][dt].z, p[b][2], o[dt], 0, 0, 0);
+        o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(vx[b][dt].w, p[b][3], o[dt], 0, 0, 0);
+      }
+  }
+  l += shfl_xor_f(l, 16);
+  l += shfl_xor_f(l, 32);
+  // the key splits' results: log-sum-exp merge by the first split's wavefront
+  // of each head (a split that saw no key of a row has m = kNegBig, l = 0, o = 0)
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<f32x4*>(&mo[wave][dt][lane][0]) = o[dt];
+  mml[wave][lane][0] = m;
+  mml[wave][lane][1] = l;
+  __syncthreads();
+  if (ks != 0 || !active || tok0 + c >= qr.len) return;
+  float mx = m;
+  for (int z = 1; z < KS; ++z) mx = fmaxf(mx, mml[z * HW + hl][lane][0]);
+  const float f0 = exp2f(m - mx);
+  l *= f0;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) o[dt] *= f0;
+  for (int z = 1; z < KS; ++z) {
+    const float f = exp2f(mml[z * HW + hl][lane][0] - mx);
+    l += mml[z * HW + hl][lane][1] * f;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+      o[dt] += *reinterpret_cast<const f32x4*>(&mo[z * HW + hl][dt][lane][0]) * f;
+  }
+  const float inv = l != 0.f ? 1.f / l : 0.f;
+  float* orow = out + ((int64_t)(qr.begin + tok0 + c) * Hq + head) * D + 4 * j;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+    *reinterpret_cast<f32x4*>(orow + 16 * dt) = o[dt] * inv;
+}
+
 // Generic: one wavefront per (query row, head); keys in chunks of 64 with
 // an online softmax; lane d accumulates output dims d, d + 64, ...
 template <typename T, typename TC = T>
@@ -1109,6 +1319,13 @@ int32_t prefill_impl(void* out, const void* q, const void* k_cache, const void* 
   const bool tiled = !kv_scales && (dtype == PA_DTYPE_BF16 || fp8) &&
                      (head_dim == 64 || head_dim == 128);
   const bool mfma = !kv_scales && dtype == PA_DTYPE_BF16 && head_dim == 256;
+  // 16-byte operand loads: rows of q and cache rows from 16-byte aligned
+  // bases (a strided view of q may start anywhere), and a grid within limits
+  const bool f32_mfma = dtype == PA_DTYPE_F32 && head_dim >= 16 && 256 % head_dim == 0 &&
+                        ((uintptr_t)q | (uintptr_t)out | (uintptr_t)k_cache |
+                         (uintptr_t)v_cache) % 16 == 0 &&
+                        q_row % 4 == 0 && num_seqs <= 65535 &&
+                        (long long)num_kv_heads * ((num_heads / num_kv_heads + 3) / 4) <= 65535;
   if (tiled) {
     const int G = num_heads / num_kv_heads;
     const int HW = G < 4 ? G : 4;
@@ -1172,6 +1389,22 @@ int32_t prefill_impl(void* out, const void* q, const void* k_cache, const void* 
       num_kv_heads, num_blocks, scale_log2, q_row, total_q, max_q_len)
     PA_LAUNCH_PREFILL(256);
 #undef PA_LAUNCH_PREFILL
+  } else if (f32_mfma) {
+    const int G = num_heads / num_kv_heads;
+    const dim3 grid((max_q_len + 15) / 16, num_kv_heads * ((G + 3) / 4), num_seqs);
+    auto launch = [&](auto dc) {
+      prefill_f32_kernel<decltype(dc)::value><<<grid, 512, 0, s>>>(
+          (float*)out, (const float*)q, (const float*)k_cache, (const float*)v_cache, block_tables,
+          max_blocks_per_seq, cu_q_lens, past_lens, num_heads, num_kv_heads, G, num_blocks,
+          scale_log2, kv_scales, q_row, total_q, max_q_len);
+    };
+    switch (head_dim) {
+      case 16: launch(IC<16>{}); break;
+      case 32: launch(IC<32>{}); break;
+      case 64: launch(IC<64>{}); break;
+      case 128: launch(IC<128>{}); break;
+      default: launch(IC<256>{}); break;
+    }
   } else {
     const dim3 grid(max_q_len, num_heads, num_seqs);
     if (dtype == PA_DTYPE_FP8_E4M3)
