@@ -21,6 +21,8 @@
 //    processed per step (32 = the MFMA K dimension of the P·V product).
 //  * decode_generic_kernel (f32 or bf16, any D <= 512, any group size): a
 //    plain reference-grade kernel, one workgroup per query head.
+#include <algorithm>
+#include <cmath>
 #include <mutex>
 #include <type_traits>
 
@@ -80,11 +82,15 @@ __device__ inline bool private_block(const int32_t* __restrict__ block_tables, i
 // through LDS, with the log-sum-exp rule of decode_reduce_kernel
 //     M = max_w m_w,  out = sum_w 2^(m_w - M) o_w / sum_w 2^(m_w - M) l_w,
 // written as the bf16 output of the group's G query heads (empty partitions
-// hold m = kNegBig, l = 0, o = 0 and drop out).  Lane (c, j) holds head c's
-// o[dt][r] for dims 16 dt + 4 j + r, as the MFMA decode kernels leave it.
+// hold m = kNegBig, l = 0, o = 0 and drop out), or, with num_parts > 1
+// workgroups per row, as partial result `part` of the rows from row0 on.  Lane
+// (c, j) holds head c's o[dt][r] for dims 16 dt + 4 j + r, as the MFMA decode
+// kernels leave it.
 template <int D, int NW>
-__device__ inline void merge_in_workgroup(uint16_t* __restrict__ out_group, const f32x4 (&o)[D / 16],
-                                          float m, float lsum, int c, int j, int G) {
+__device__ inline void merge_in_workgroup(uint16_t* __restrict__ out, const f32x4 (&o)[D / 16],
+                                          float m, float lsum, int c, int j, int G, int64_t row0,
+                                          int part, int num_parts, float* __restrict__ ws_o,
+                                          float* __restrict__ ws_ml) {
   __shared__ float so[NW][16][D];
   __shared__ float sml[NW][16][2];
   const int wave = threadIdx.x >> 6;
@@ -111,9 +117,45 @@ __device__ inline void merge_in_workgroup(uint16_t* __restrict__ out_group, cons
       num += a * so[w][hc][d];
       den += a * sml[w][hc][1];
     }
-    // den is 0 only for a row with no keys; a NaN den (a NaN score) must
-    // reach the output, so the test is != 0, not > 0
-    out_group[idx] = f32_to_bf16_bits(den != 0.f ? num / den : 0.f);
+    if (num_parts == 1) {
+      // den is 0 only for a row with no keys; a NaN den (a NaN score) must
+      // reach the output, so the test is != 0, not > 0
+      out[row0 * D + idx] = f32_to_bf16_bits(den != 0.f ? num / den : 0.f);
+    } else {
+      const int64_t at = (row0 + hc) * num_parts + part;
+      ws_o[at * D + d] = num;
+      if (d == 0) {
+        ws_ml[2 * at] = mx;
+        ws_ml[2 * at + 1] = den;
+      }
+    }
+  }
+}
+
+// The tokens of partition `part`: part_len from part * part_len, or, with
+// part_len 0 (NW > 1), an equal share of the context's 32-token steps among
+// the NW wavefronts of the row's num_parts workgroups, whatever its length
+// (fixed partitions, sized for the launch's longest context, leave most
+// wavefronts of the shorter ones idle; those of 128 tokens, at most 8 of them,
+// stay fixed: 32 x 192-640 tokens over 2 kv heads 7.3 us, 7.6 in shares).
+struct TokenRange {
+  int begin, end;
+};
+template <int NW>
+__device__ inline TokenRange token_range(int ctx, int part, int num_parts, int part_len) {
+  if (NW == 1 || part_len > 0) {
+    return {part * part_len, min(ctx, (part + 1) * part_len)};
+  } else {
+    // the workgroup's share, then the wavefront's of that (quotients by the
+    // constant NW; steps < 2^26 and at most 32 workgroups)
+    int a = 0, b = (max(ctx, 0) + 2 * kBlock - 1) / (2 * kBlock);
+    if (num_parts > 1) {
+      const uint32_t steps = b, x = part / NW;
+      a = x * steps / num_parts;
+      b = (x + 1) * steps / num_parts;
+    }
+    const int n = b - a, w = part % NW;
+    return {(a + w * n / NW) * 2 * kBlock, min(ctx, (a + (w + 1) * n / NW) * 2 * kBlock)};
   }
 }
 
@@ -141,29 +183,15 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     float* __restrict__ ws_ml, int64_t q_row, const uint8_t* /* FP8 flags, unused */) {
   constexpr int KS = D / 32;  // QK reduction steps
   constexpr int DT = D / 16;  // PV output tiles
-  // NW > 1: the workgroup's wavefronts take partitions blockIdx.x * NW + w
-  // (the launch uses it only when one workgroup holds all of them) and merge
-  // them in LDS; NW = 1: one partition, merged by decode_reduce_kernel.
+  // NW > 1: the wavefronts of num_parts workgroups share the context
+  // (token_range); a workgroup's merge in LDS, several workgroups' results in
+  // decode_reduce_kernel.  NW = 1: one partition, merged by that kernel.
   const int lane = threadIdx.x & 63;
   const int c = lane & 15, j = lane >> 4;
   const int part = blockIdx.x * NW + (NW > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0);
   const int kvh = blockIdx.y, seq = blockIdx.z;
-  // Clamp to what the block table can address so a bad length never reads
-  // past the table.
-  const int ctx = min(context_lens[seq], mbs * kBlock);
-  const int tok0 = part * part_len;
-  const bool empty = tok0 >= ctx;
-  if (NW == 1 && empty) {
-    // Empty context: the output is defined as zeros.
-    if (num_parts == 1 && c < G) {
-      uint16_t* orow = out + ((int64_t)seq * Hq + kvh * G + c) * D;
-      for (int d = 4 * j; d < D; d += 16) *reinterpret_cast<uint64_t*>(orow + d) = 0;
-    }
-    return;
-  }
-  const int tok_end = empty ? tok0 : min(ctx, tok0 + part_len);
-  const int nblk = (tok_end - tok0 + kBlock - 1) / kBlock;  // 0 for an empty partition
-
+  // the query rows first: their loads are in flight while the context length
+  // arrives (waited for before them, a short launch took 3% longer)
   const int head = kvh * G + c;
   bf16x8 qv[KS];
 #pragma unroll
@@ -173,6 +201,23 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     else
       qv[s] = bf16x8{};
   }
+  // Clamp to what the block table can address so a bad length never reads
+  // past the table.
+  const int ctx = min(context_lens[seq], mbs * kBlock);
+  const TokenRange tr = token_range<NW>(ctx, part, num_parts, part_len);
+  const int tok0 = __builtin_amdgcn_readfirstlane(tr.begin);
+  const int tr_end = __builtin_amdgcn_readfirstlane(tr.end);
+  const bool empty = tok0 >= tr_end;
+  if (NW == 1 && empty) {
+    // Empty context: the output is defined as zeros.
+    if (num_parts == 1 && c < G) {
+      uint16_t* orow = out + ((int64_t)seq * Hq + kvh * G + c) * D;
+      for (int d = 4 * j; d < D; d += 16) *reinterpret_cast<uint64_t*>(orow + d) = 0;
+    }
+    return;
+  }
+  const int tok_end = empty ? tok0 : tr_end;
+  const int nblk = (tok_end - tok0 + kBlock - 1) / kBlock;  // 0 for an empty partition
 
   f32x4 o[DT];
 #pragma unroll
@@ -330,7 +375,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
   lsum += shfl_xor_f(lsum, 16);
   lsum += shfl_xor_f(lsum, 32);
   if constexpr (NW > 1) {
-    merge_in_workgroup<D, NW>(out + ((int64_t)seq * Hq + kvh * G) * D, o, m, lsum, c, j, G);
+    merge_in_workgroup<D, NW>(out, o, m, lsum, c, j, G, (int64_t)seq * Hq + kvh * G, blockIdx.x,
+                              num_parts, ws_o, ws_ml);
     return;
   }
   if (c >= G) return;
@@ -573,16 +619,24 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(D <= 12
   constexpr int KS = Part::KS;
   constexpr int DT = Part::DT;
   constexpr int DL = Part::DL;
-  // NW > 1: the workgroup's wavefronts take partitions blockIdx.x * NW + w
-  // (the launch uses it only when one workgroup holds all of them) and merge
-  // them in LDS; NW = 1: one partition, merged by decode_reduce_kernel.
+  // NW > 1: the wavefronts of num_parts workgroups share the context
+  // (token_range); a workgroup's merge in LDS, several workgroups' results in
+  // decode_reduce_kernel.  NW = 1: one partition, merged by that kernel.
   const int lane = threadIdx.x & 63;
   const int c = lane & 15, j = lane >> 4;
   const int part = blockIdx.x * NW + (NW > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0);
   const int kvh = blockIdx.y, seq = blockIdx.z;
+  const int head = kvh * G + c;
+  const uint16_t* qrow = c < G ? q + (int64_t)seq * q_row + (int64_t)head * D : nullptr;
+  bf16x8 qv[KS];
+#pragma unroll
+  for (int s = 0; s < KS; ++s)
+    qv[s] = qrow ? *reinterpret_cast<const bf16x8*>(qrow + DL * j + 8 * s) : bf16x8{};
   const int ctx = min(context_lens[seq], mbs * kBlock);
-  const int tok0 = part * part_len;
-  const bool empty = tok0 >= ctx;
+  const TokenRange tr = token_range<NW>(ctx, part, num_parts, part_len);
+  const int tok0 = __builtin_amdgcn_readfirstlane(tr.begin);
+  const int tr_end = __builtin_amdgcn_readfirstlane(tr.end);
+  const bool empty = tok0 >= tr_end;
   if (NW == 1 && empty) {
     if (num_parts == 1 && c < G) {
       uint16_t* orow = out + ((int64_t)seq * Hq + kvh * G + c) * D;
@@ -590,17 +644,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(D <= 12
     }
     return;
   }
-  const int tok_end = empty ? tok0 : min(ctx, tok0 + part_len);
+  const int tok_end = empty ? tok0 : tr_end;
   const Part P{kc, vc, block_tables + (int64_t)seq * mbs + tok0 / kBlock, Hkv, kvh, num_blocks,
                tok0, tok_end, (tok_end - tok0 + kBlock - 1) / kBlock /* 0 when empty */, c, j,
                scale_log2, block_flags};
 
-  const int head = kvh * G + c;
-  const uint16_t* qrow = c < G ? q + (int64_t)seq * q_row + (int64_t)head * D : nullptr;
-  bf16x8 qv[KS];
-#pragma unroll
-  for (int s = 0; s < KS; ++s)
-    qv[s] = qrow ? *reinterpret_cast<const bf16x8*>(qrow + DL * j + 8 * s) : bf16x8{};
   typename Part::State S;
   P.init(S);
 
@@ -642,7 +690,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(D <= 12
   lsum += shfl_xor_f(lsum, 16);
   lsum += shfl_xor_f(lsum, 32);
   if constexpr (NW > 1) {
-    merge_in_workgroup<D, NW>(out + ((int64_t)seq * Hq + kvh * G) * D, S.o, S.m, lsum, c, j, G);
+    merge_in_workgroup<D, NW>(out, S.o, S.m, lsum, c, j, G, (int64_t)seq * Hq + kvh * G,
+                              blockIdx.x, num_parts, ws_o, ws_ml);
     return;
   }
   if (c >= G) return;
@@ -1423,7 +1472,7 @@ __global__ __launch_bounds__(256) void decode_reduce_kernel(
     int part_len, int balance_nw, int B, int Hkv, const int32_t* __restrict__ grp, int cap) {
   // balance_nw > 0: partial results of decode_balanced_kernel launched with
   // balance_nw wavefronts (num_parts = slots per row; grp its groups);
-  // else partitions of part_len tokens.
+  // else partitions of part_len tokens (0: equal shares of every context).
   __shared__ float red[4][64 * kDL];
   __shared__ float wml[2][4];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -1453,7 +1502,8 @@ __global__ __launch_bounds__(256) void decode_reduce_kernel(
                num_parts);
     }
   } else {
-    np = min(num_parts, (ctx + part_len - 1) / part_len);
+    // (part_len 0: every workgroup of the row wrote a result)
+    np = ctx <= 0 ? 0 : part_len > 0 ? min(num_parts, (ctx + part_len - 1) / part_len) : num_parts;
   }
   const int64_t row0 = (int64_t)row * num_parts;
   constexpr int kRU = 8;
@@ -1541,6 +1591,47 @@ int choose_partition(int num_seqs, int num_kv_heads, int max_ctx, int head_dim, 
   return kPart;
 }
 
+// Workgroups per (kv head, sequence) whose results the reduce kernel merges,
+// for launches whose wavefronts merge in LDS.  One workgroup streams at most
+// about 43 GB/s (bf16; FP8, with one step in flight per wavefront, 36; 36 / 31
+// with 32 of them running, 29 / 25 with 128), so few (kv head, sequence) pairs leave the
+// chip idle, and a number of them that does not fill whole rounds of the 256
+// CUs leaves it idle in the last.  More workgroups cost the reduce launch
+// (3.2 us) and 1.4% of the stream each.  Estimated over the launch's longest
+// context for every sequence (the others' are on the device); the least
+// wins, one workgroup where they tie.  Measured, us, one workgroup / chosen:
+// bf16, 8 kv heads x 128: 1 x 2000 tokens 27.0 / 10.0, 1 x 500 9.8 / 7.5, 4 x
+// 2000 32.1 / 11.3, 16 x 200-2000 27.3 / 19.6, 48 x 4096 157 / 132, 37 x
+// 500-8000 120 / 91, 64 x 4096 170 / 170 (one; two workgroups 175); FP8: 37 x
+// 500-8000 69 / 56, 16 x 8000 78 / 50, 1 x 2000 19 / 9.
+int choose_splits(int num_seqs, int num_heads, int num_kv_heads, int head_dim, int max_ctx,
+                  int elem_bytes, size_t workspace_bytes) {
+  constexpr double kCUs = 256;
+  const double pairs = (double)num_seqs * num_kv_heads;
+  const double pair_us = 2e-3 * max_ctx * head_dim * elem_bytes;  // bytes / 1000: us at 1 GB/s
+  const double all = elem_bytes == 1 ? 6200. : 6500.;
+  auto one = [&](double wgs) {
+    return (elem_bytes == 1 ? 36. : 43.) * (wgs <= 16 ? 1. : wgs <= 64 ? 0.85 : 0.68);
+  };
+  int best = 1;
+  double best_us = 0.;
+  for (int s : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32}) {
+    const double wgs = pairs * s;
+    if (s > 1 && (max_ctx < 64 * s || wgs > 4096. ||
+                  (size_t)num_seqs * num_heads * s * (head_dim + 2) * sizeof(float) >
+                      workspace_bytes))
+      break;
+    const double rounds = wgs <= kCUs ? 1. : std::ceil(wgs / kCUs) * kCUs / wgs;
+    double us = std::max(pairs * pair_us / all * rounds, wgs <= kCUs ? pair_us / s / one(wgs) : 0.);
+    if (s > 1) us = us * (1. + 0.014 * s) + 3.2;
+    if (s == 1 || us < best_us) {
+      best = s;
+      best_us = us;
+    }
+  }
+  return best;
+}
+
 }  // namespace
 }  // namespace pa
 
@@ -1567,10 +1658,12 @@ struct DecodePlan {
   bool balanced;  // bf16 launches that would need the reduce: decode_balanced_kernel
   int share_sp;   // balanced: sequences per shared-prefix group (1: no sharing)
   int part_len, np, merge_waves;  // np: partitions, or partial-result slots per row
+  int splits;     // merge_waves > 1: workgroups per (kv head, sequence)
   size_t ws_bytes;  // workspace the launch needs (0: none)
 };
 DecodePlan decode_plan(int32_t dtype, bool quantized, int32_t num_seqs, int32_t num_heads,
-                       int32_t num_kv_heads, int32_t head_dim, int32_t max_context_len) {
+                       int32_t num_kv_heads, int32_t head_dim, int32_t max_context_len,
+                       size_t workspace_bytes) {
   DecodePlan p{};
   const int G = num_heads / num_kv_heads;
   const bool fp8 = dtype == PA_DTYPE_FP8_E4M3;
@@ -1597,6 +1690,11 @@ DecodePlan decode_plan(int32_t dtype, bool quantized, int32_t num_seqs, int32_t 
                   : p.np <= 4           ? 4
                   : (p.np <= 8 && head_dim <= 128) ? 8
                                                    : 1;
+  // FP8 contexts of more partitions than that: eight wavefronts share them
+  if (fp8 && p.mfma && p.np > 1 && p.merge_waves == 1) p.merge_waves = head_dim <= 128 ? 8 : 4;
+  p.splits = p.merge_waves > 1 ? choose_splits(num_seqs, num_heads, num_kv_heads, head_dim,
+                                               max_context_len, fp8 ? 1 : 2, workspace_bytes)
+                               : 1;
   // Partitioned launches that need the reduce (long, ragged contexts) cut
   // the work evenly over the GPU instead (bf16 caches).
   p.balanced = p.mfma && !fp8 && p.np > 1 && p.merge_waves == 1;
@@ -1615,7 +1713,8 @@ DecodePlan decode_plan(int32_t dtype, bool quantized, int32_t num_seqs, int32_t 
     p.np = (max_units + kBalanceMinUnits - 1) / kBalanceMinUnits + 3;
     if (G <= 8 && num_seqs >= 2 && num_seqs <= kGroupMaxSeqs) p.share_sp = 16 / G;
   }
-  p.ws_bytes = p.np > 1 && p.merge_waves == 1
+  if (p.merge_waves > 1) p.np = p.splits;
+  p.ws_bytes = p.np > 1
                    ? (size_t)num_seqs * num_heads * p.np * (head_dim + 2) * sizeof(float) +
                          (p.share_sp > 1 ? (6 * (size_t)num_seqs + 2) * sizeof(int32_t) : 0)
                    : 0;
@@ -1645,11 +1744,15 @@ int32_t decode_impl(void* out, const void* q, const void* k_cache, const void* v
   PA_REQUIRE(out && q && k_cache && v_cache && block_tables && context_lens, PA_ERR_INVALID_ARG,
              "pa_decode: null pointer");
   const DecodePlan plan = decode_plan(dtype, kv_scales != nullptr, num_seqs, num_heads,
-                                      num_kv_heads, head_dim, max_context_len);
+                                      num_kv_heads, head_dim, max_context_len,
+                                      workspace ? workspace_bytes : 0);
   const int G = num_heads / num_kv_heads;
   const bool fp8 = dtype == PA_DTYPE_FP8_E4M3;
   const bool mfma = plan.mfma, f32_group = plan.f32_group;
-  const int part_len = plan.part_len, np = plan.np, merge_waves = plan.merge_waves;
+  const int np = plan.np, merge_waves = plan.merge_waves;
+  // 0: equal shares
+  const int part_len =
+      merge_waves > 1 && (np > 1 || plan.part_len > kPart / 2) ? 0 : plan.part_len;
   PA_REQUIRE(np <= 1024, PA_ERR_UNSUPPORTED,
              "pa_decode: context of %d tokens needs %d > 1024 partitions", max_context_len, np);
   float* ws_o = nullptr;
@@ -1687,7 +1790,7 @@ int32_t decode_impl(void* out, const void* q, const void* k_cache, const void* v
       PA_LAUNCH_BALANCED(256);
 #undef PA_LAUNCH_BALANCED
   } else if (mfma) {
-    const dim3 grid(merge_waves > 1 ? 1 : np, num_kv_heads, num_seqs);
+    const dim3 grid(np, num_kv_heads, num_seqs);
     auto* o = (uint16_t*)out;
     auto* qq = (const uint16_t*)q;
 #define PA_LAUNCH_MFMA_NW(KERNEL, TC, DD, NW, ...)                                            \
@@ -1767,7 +1870,7 @@ int32_t decode_impl(void* out, const void* q, const void* k_cache, const void* v
           num_blocks, scale_log2, np, ws_o, ws_ml, kv_scales, q_row);
   }
   int32_t rc = check_launch("pa_decode");
-  if (rc != PA_OK || np == 1 || merge_waves > 1) return rc;
+  if (rc != PA_OK || np == 1) return rc;
   const dim3 rgrid(num_seqs * num_heads);
   const int bal = plan.balanced ? kBalanceWaves : 0;
 #define PA_LAUNCH_REDUCE(TT, DL)                                                              \
@@ -1908,7 +2011,7 @@ extern "C" int32_t pa_decode_noalloc(void* out, const void* q, const void* k_cac
   if (num_seqs > 0 && num_heads > 0 && num_kv_heads > 0 && head_dim > 0 &&
       num_heads % num_kv_heads == 0 && max_context_len > 0) {
     const DecodePlan plan = decode_plan(dtype, false, num_seqs, num_heads, num_kv_heads,
-                                        head_dim, max_context_len);
+                                        head_dim, max_context_len, kDecodeScratchBytes);
     PA_REQUIRE(plan.ws_bytes <= kDecodeScratchBytes, PA_ERR_WORKSPACE,
                "pa_decode_noalloc: %d sequences x %d heads at context %d need %zu bytes of "
                "split-K scratch, above the fixed %zu (use pa_decode with a workspace)",
