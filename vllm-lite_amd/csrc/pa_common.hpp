@@ -134,10 +134,14 @@ __host__ __device__ inline float bf16_bits_to_f32(uint16_t h) {
   return __builtin_bit_cast(float, (uint32_t)h << 16);
 }
 __host__ __device__ inline uint16_t f32_to_bf16_bits(float f) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return __builtin_bit_cast(uint16_t, (__bf16)f);  // v_cvt_pk_bf16_f32, nearest even too
+#else
   uint32_t u = __builtin_bit_cast(uint32_t, f);
   if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40);
   u += 0x7fffu + ((u >> 16) & 1u);
   return (uint16_t)(u >> 16);
+#endif
 }
 
 // Element access for the two storage types.
