@@ -145,10 +145,12 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_kernel(
 #pragma unroll
     for (int u = 0; u < CB; ++u) lds_copy16(wb[u] + (int64_t)kt * RB, wo[u], lb + u * 1024);
   };
-  if constexpr (EPI == 1) {
-    for (int i = threadIdx.x; i < BN; i += NT) sbias[i] = bf16_bits_to_f32(bias[min(c0 + i, N - 1)]);
-    wait_copies<0>();  // the steps' waits count copies only
-  }
+  // the tile's bias: loaded here, put into LDS after the steps (a wait for it
+  // here would come before the first copy; older than the copies, it does not
+  // disturb the steps' counts)
+  static_assert(EPI != 1 || NT >= BN, "one bias value per thread");
+  uint16_t bias_raw = 0;
+  if (EPI == 1 && threadIdx.x < BN) bias_raw = bias[min(c0 + (int)threadIdx.x, N - 1)];
   // LDS rows of this wavefront's operand tiles (SwiGLU: gate tiles, then the
   // matching up tiles)
   int arow[TM], brow[TN];
@@ -205,6 +207,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_kernel(
     buf = buf == S - 1 ? 0 : buf + 1;
     ibuf = ibuf == S - 1 ? 0 : ibuf + 1;
   }
+  if (EPI == 1 && threadIdx.x < BN) sbias[threadIdx.x] = bf16_bits_to_f32(bias_raw);
   __syncthreads();
   // the K groups' sums, in group order
   if constexpr (KG > 1) {
@@ -364,7 +367,7 @@ Tiling choose_tiling(int M, int wrows, int K, bool silu) {
     int bm, bn;
     float us, ns_per_k;
   };
-  static constexpr Cost costs[] = {{k256x256, 256, 256, 6.5f, 25.7f}, {k256x128, 256, 128, 5.f, 15.f},
+  static constexpr Cost costs[] = {{k256x256, 256, 256, 6.5f, 25.7f}, {k256x128, 256, 128, 5.5f, 15.f},
                                    {k128x128, 128, 128, 3.4f, 8.2f},  {k64x128, 64, 128, 4.f, 4.9f},
                                    {k64x64, 64, 64, 3.1f, 2.6f}};
   auto tiles = [&](int bm, int bn) {
@@ -372,13 +375,20 @@ Tiling choose_tiling(int M, int wrows, int K, bool silu) {
   };
   Tiling best = k128x128;
   double best_us = 1e30;
-  // more 128 x 128 tiles than CUs: two workgroups share a CU, and whichever
-  // finishes is replaced, so rounds are fractional (SwiGLU stores half as
-  // many outputs per tile: 134.6 us against 256 x 256's 137.9 at 7160 x 9728,
-  // where the plain epilogue loses, 236.7 against 202.0 at 640 x 151936 x 896)
-  if (tiles(128, 128) > kCUs) {
+  // More 128 x 128 tiles than CUs: two workgroups share a CU, and whichever
+  // finishes is replaced.  The last round runs one tile per CU where it is at
+  // most half full (540 tiles, K 896, with bias: 30.7 us against 20 for 504 and
+  // 26 in 256 x 256).  (SwiGLU stores half as many outputs per tile: 134.6 us
+  // against 256 x 256's 137.9 at 7160 x 9728, where the plain epilogue loses,
+  // 236.7 against 202.0 at 640 x 151936 x 896.)
+  const double pair = (silu ? 3. : 4.) + 15.5e-3 * K, alone = 3. + 8.4e-3 * K;
+  if (const double n = tiles(128, 128); n > kCUs) {
+    const double full = std::floor(n / (2 * kCUs)), rest = n - full * 2 * kCUs;
     best = k128x128Pair;
-    best_us = 4. + tiles(128, 128) / (2 * kCUs) * ((silu ? 3. : 4.5) + 15.3e-3 * K);
+    best_us = 3.5 + full * pair +
+              (rest == 0. ? 0.
+               : rest <= kCUs ? alone
+                              : std::max(rest / (2 * kCUs), full > 0. ? 0. : 0.85) * pair);
   }
   for (const Cost& c : costs) {
     const double us = std::ceil(tiles(c.bm, c.bn) / kCUs) * (c.us + c.ns_per_k * 1e-3 * K);
