@@ -331,6 +331,38 @@ __global__ __launch_bounds__(256) void read_kv_kernel(const T* __restrict__ k_ca
   }
 }
 
+// The same for D <= kReadMaxD, one workgroup per block and head: the K rows in
+// order, the token-minor V block read in order and turned through LDS (element
+// by element, a token's V read touched 32 bytes for each 2 or 4 it used).
+constexpr int kReadMaxD = 512;
+template <typename T, typename Ids>
+__global__ __launch_bounds__(256) void read_kv_block_kernel(const T* __restrict__ k_cache,
+                                                            const T* __restrict__ v_cache,
+                                                            Ids block_ids, int seq_len, int H,
+                                                            int D, int num_blocks,
+                                                            T* __restrict__ out_k,
+                                                            T* __restrict__ out_v) {
+  __shared__ T vt[kReadMaxD * (kBlock + 1)];
+  const int b = blockIdx.x, h = blockIdx.y;
+  int32_t blk;
+  if constexpr (std::is_pointer_v<Ids>)
+    blk = block_ids[b];
+  else
+    blk = block_ids.id[b];
+  const bool ok = blk >= 0 && blk < num_blocks;
+  const int64_t src = ((int64_t)(ok ? blk : 0) * H + h) * kBlock * D;
+  const int n = min(kBlock, seq_len - b * kBlock);
+  for (int i = threadIdx.x; i < kBlock * D; i += 256)
+    vt[i / kBlock * (kBlock + 1) + i % kBlock] = ok ? v_cache[src + i] : T(0);
+  __syncthreads();
+  for (int i = threadIdx.x; i < n * D; i += 256) {
+    const int j = i / D, d = i % D;
+    const int64_t dst = ((int64_t)(b * kBlock + j) * H + h) * D + d;
+    out_k[dst] = ok ? k_cache[src + i] : T(0);
+    out_v[dst] = vt[d * (kBlock + 1) + j];
+  }
+}
+
 // write_kv of one token (buffer.rs:103-267) in one launch: the hash of the K
 // block as it stands after the token (buffer.rs:263-264; the token's rows
 // from the input, the others from the cache), then the token's K row and V
@@ -362,39 +394,78 @@ __global__ __launch_bounds__(256) void write_token_kernel(T* __restrict__ k_cach
   }
 }
 
+// The part of a block's hash that one token row (slot `slot`, all heads)
+// contributes: sum of term(val(hd, dd)) 31^(n - 1 - e) over its elements e =
+// (hd 16 + slot) D + dd, mod 2^64, by the 16 lanes k = 0 .. 15 of a row (dims
+// k, k + 16, ...); lane 0 returns it.  Every lane of the wavefront calls it.
+template <typename F>
+__device__ inline uint64_t row_hash(int H, int D, int slot, int k, bool on, F val) {
+  uint64_t acc = 0;
+  if (on && k < D) {
+    const int last = (D - 1 - k) / 16;  // this lane's last dim k + 16 last
+    // from the last head's last dim (the smallest exponent) backwards
+    uint64_t p = pow_u64(31u, (uint64_t)((kBlock - 1 - slot) * D + D - 1 - (k + 16 * last)));
+    const uint64_t step = pow_u64(31u, 16u);
+    const uint64_t next_head = pow_u64(31u, (uint64_t)(kBlock * D - 16 * last));
+    for (int hd = H - 1; hd >= 0; --hd) {
+      for (int x = last; x >= 0; --x) {
+        acc += hash_term(val(hd, k + 16 * x)) * p;
+        if (x > 0) p *= step;
+      }
+      p *= next_head;
+    }
+  }
+#pragma unroll
+  for (int w = 8; w > 0; w >>= 1) acc += __shfl_xor((unsigned long long)acc, w, 64);
+  return acc;
+}
+
 // The reference's block-hash bookkeeping of a write (buffer.rs:263-264):
 // after every token written, the hash of the K block it landed in.  Runs
 // before the scatter of the same tokens, on the cache as it was before the
-// call: one workgroup per block task walks the task's tokens in order; per
-// token, slot o's rows come from the token that last wrote slot o in this
-// call (last[o]), the other slots from the cache; hashes[tok[i]] is the
-// hash after token tok[i] (tokens in call order).
+// call: one workgroup per block task; hashes[tok[i]] is the hash after token
+// tok[i] (tokens in call order).  The hash is a sum over the block's 16 token
+// rows, so a token changes it by its row's part minus the part of the row it
+// replaces: the rows' parts, old and new, are formed once, 16 at a time, and
+// the running sum gives every hash (hashing the whole block after every token
+// took 63 us for 1000 tokens of 2 heads x 64, f32; here 11.7).
 template <typename T>
 __global__ __launch_bounds__(256) void block_hash_replay_kernel(
     const T* __restrict__ k_cache, const T* __restrict__ key, int H, int D,
     const int32_t* __restrict__ task_block, const int32_t* __restrict__ task_beg,
     const int32_t* __restrict__ tok, const int32_t* __restrict__ off,
     uint64_t* __restrict__ hashes) {
-  __shared__ uint64_t red[256];
-  __shared__ int last[kBlock];
-  const int w = blockIdx.x;
-  const int n = H * kBlock * D;
-  const T* base = k_cache + (int64_t)task_block[w] * n;
-  if (threadIdx.x < kBlock) last[threadIdx.x] = -1;
-  __syncthreads();
-  for (int i = task_beg[w]; i < task_beg[w + 1]; ++i) {
-    if (threadIdx.x == 0) last[off[i]] = tok[i];
+  __shared__ uint64_t part[kBlock], fresh[kBlock];
+  __shared__ int to[kBlock], oo[kBlock];
+  const int w = blockIdx.x, r = threadIdx.x >> 4, k = threadIdx.x & 15;
+  const T* base = k_cache + (int64_t)task_block[w] * H * kBlock * D;
+  const int beg = task_beg[w], end = task_beg[w + 1];
+  const uint64_t old = row_hash(H, D, r, k, true, [&](int hd, int dd) -> float {
+    return Elem<T>::load(base + ((int64_t)hd * kBlock + r) * D + dd);
+  });
+  if (k == 0) part[r] = old;
+  for (int i0 = beg; i0 < end; i0 += kBlock) {
+    const bool on = i0 + r < end;
+    const int t = on ? tok[i0 + r] : 0, o = on ? off[i0 + r] : 0;
+    const uint64_t c = row_hash(H, D, o, k, on, [&](int hd, int dd) -> float {
+      return Elem<T>::load(key + ((int64_t)t * H + hd) * D + dd);
+    });
+    if (k == 0) {
+      fresh[r] = c;
+      to[r] = t;
+      oo[r] = o;
+    }
     __syncthreads();
-    const uint64_t h = workgroup_block_hash(
-        n,
-        [&](int e) -> float {
-          const int hd = e / (kBlock * D), r = e % (kBlock * D);
-          const int j = last[r / D];
-          return j >= 0 ? Elem<T>::load(key + ((int64_t)j * H + hd) * D + r % D)
-                        : Elem<T>::load(base + e);
-        },
-        red);
-    if (threadIdx.x == 0) hashes[tok[i]] = h;
+    if (threadIdx.x == 0) {
+      uint64_t total = 0;
+      for (int j = 0; j < kBlock; ++j) total += part[j];
+      for (int j = 0; j < min(kBlock, end - i0); ++j) {
+        total += fresh[j] - part[oo[j]];
+        part[oo[j]] = fresh[j];
+        hashes[to[j]] = total;
+      }
+    }
+    __syncthreads();
   }
 }
 
@@ -447,19 +518,34 @@ int32_t launch_write_token(void* k_cache, void* v_cache, const void* key, const 
   return check_launch("write_kv");
 }
 
+namespace {
+template <typename Ids>
+void launch_read(const void* k_cache, const void* v_cache, int32_t dtype, const Ids& ids,
+                 int seq_len, int H, int D, int num_blocks, void* out_k, void* out_v,
+                 hipStream_t s) {
+  auto go = [&](auto elem) {
+    using T = decltype(elem);
+    if (D <= kReadMaxD && H <= 65535)
+      read_kv_block_kernel<T, Ids><<<dim3((seq_len + kBlock - 1) / kBlock, H), 256, 0, s>>>(
+          (const T*)k_cache, (const T*)v_cache, ids, seq_len, H, D, num_blocks, (T*)out_k,
+          (T*)out_v);
+    else
+      read_kv_kernel<T, Ids><<<seq_len, 256, 0, s>>>((const T*)k_cache, (const T*)v_cache, ids, H,
+                                                     D, num_blocks, (T*)out_k, (T*)out_v);
+  };
+  if (dtype == PA_DTYPE_BF16)
+    go(uint16_t{});
+  else
+    go(float{});
+}
+}  // namespace
+
 int32_t launch_read_kv_small(const void* k_cache, const void* v_cache, int32_t dtype,
                              const int32_t* ids, int n_ids, int seq_len, int H, int D,
                              int num_blocks, void* out_k, void* out_v, hipStream_t stream) {
   SmallIds v{};
   for (int i = 0; i < n_ids && i < kSmallIds; ++i) v.id[i] = ids[i];
-  if (dtype == PA_DTYPE_BF16)
-    read_kv_kernel<uint16_t, SmallIds><<<seq_len, 256, 0, stream>>>(
-        (const uint16_t*)k_cache, (const uint16_t*)v_cache, v, H, D, num_blocks,
-        (uint16_t*)out_k, (uint16_t*)out_v);
-  else
-    read_kv_kernel<float, SmallIds><<<seq_len, 256, 0, stream>>>(
-        (const float*)k_cache, (const float*)v_cache, v, H, D, num_blocks, (float*)out_k,
-        (float*)out_v);
+  launch_read(k_cache, v_cache, dtype, v, seq_len, H, D, num_blocks, out_k, out_v, stream);
   return check_launch("read_kv");
 }
 
@@ -669,14 +755,9 @@ extern "C" int32_t pa_read_kv(const void* k_cache, const void* v_cache, const in
     read_kv_fp8_kernel<<<seq_len, 256, 0, s>>>(
         (const uint8_t*)k_cache, (const uint8_t*)v_cache, block_ids, num_kv_heads, head_dim,
         num_blocks, (float*)out_k, (float*)out_v);
-  else if (dtype == PA_DTYPE_BF16)
-    read_kv_kernel<uint16_t, const int32_t*><<<seq_len, 256, 0, s>>>(
-        (const uint16_t*)k_cache, (const uint16_t*)v_cache, block_ids, num_kv_heads, head_dim,
-        num_blocks, (uint16_t*)out_k, (uint16_t*)out_v);
   else
-    read_kv_kernel<float, const int32_t*><<<seq_len, 256, 0, s>>>(
-        (const float*)k_cache, (const float*)v_cache, block_ids, num_kv_heads, head_dim,
-        num_blocks, (float*)out_k, (float*)out_v);
+    launch_read(k_cache, v_cache, dtype, block_ids, seq_len, num_kv_heads, head_dim, num_blocks,
+                out_k, out_v, s);
   return check_launch("pa_read_kv");
 }
 
