@@ -11,9 +11,7 @@
 
 #include <algorithm>
 #include <cstring>
-#include <map>
 #include <unordered_map>
-#include <unordered_set>
 #include <vector>
 
 #include "../../include/pa_kv_cache.h"
@@ -32,23 +30,38 @@ struct pa_kv_cache {
   void* host_stage = nullptr;
   void* dev_stage = nullptr;
   size_t stage_bytes = 0;
-  // One token's block hash, written by the device into host-mapped memory
-  // (write_kv of a single token: no index upload, no copy back).
+  // The block hashes of a write's tokens, written by the device into
+  // host-mapped memory (nothing to copy back).
   uint64_t* hash_host = nullptr;
   uint64_t* hash_dev = nullptr;
+  size_t hash_slots = 0;
+  // A write's grouping by block: each block's task in the call (-1 between
+  // calls), and per task the place of its next token and the slots written.
+  struct Task {
+    int32_t next;
+    uint32_t written;
+  };
+  std::vector<int32_t> block_task;
+  std::vector<Task> task_slots;
 
-  int32_t ensure_hash_slot() {
-    if (hash_host) return PA_OK;
+  int32_t ensure_hash_slots(size_t count) {
+    if (count <= hash_slots) return PA_OK;
+    if (hash_host) (void)hipHostFree(hash_host);
+    hash_host = hash_dev = nullptr;
+    hash_slots = 0;
+    const size_t cap = count < 32 ? 32 : count;
     void* h = nullptr;
     void* d = nullptr;
-    if (hipHostMalloc(&h, 256, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
+    if (hipHostMalloc(&h, cap * sizeof(uint64_t), hipHostMallocMapped | hipHostMallocCoherent) !=
+            hipSuccess ||
         hipHostGetDevicePointer(&d, h, 0) != hipSuccess) {
       if (h) (void)hipHostFree(h);
-      pa::set_error("pa_kv_cache: allocating the mapped hash slot failed");
+      pa::set_error("pa_kv_cache: allocating %zu mapped hash slots failed", cap);
       return PA_ERR_HIP;
     }
     hash_host = (uint64_t*)h;
     hash_dev = (uint64_t*)d;
+    hash_slots = cap;
     return PA_OK;
   }
 
@@ -72,13 +85,11 @@ struct pa_kv_cache {
     return PA_OK;
   }
 
-  // Copies `bytes` of host data to the device stage on `stream` and returns
-  // the device pointer.  The caller synchronises the stream before the
-  // stage is reused.
-  void* upload(const void* src, size_t bytes, hipStream_t stream, int32_t* rc) {
-    *rc = ensure_stage(bytes);
-    if (*rc != PA_OK) return nullptr;
-    std::memcpy(host_stage, src, bytes);
+  // Copies the first `bytes` of the pinned stage, filled by the caller after
+  // ensure_stage, to the device stage on `stream` and returns the device
+  // pointer.  The caller synchronises the stream before the stage is reused.
+  void* upload(size_t bytes, hipStream_t stream, int32_t* rc) {
+    *rc = PA_OK;
     if (hipMemcpyAsync(dev_stage, host_stage, bytes, hipMemcpyHostToDevice, stream) !=
         hipSuccess) {
       pa::set_error("pa_kv_cache: index upload failed");
@@ -112,69 +123,77 @@ int32_t finish(hipStream_t stream, int32_t rc) {
 // the hashes are replayed from the cache before the scatter (one kernel),
 // then the tokens are scattered; quantised caches: each block is
 // re-quantised once per token (quant_write_kernel), which also hashes it.
+//
+// The grouping is two passes over the tokens with a table of the cache's
+// blocks (std::map and unordered_set per call took about 50 us for 1000
+// tokens), built in the pinned stage itself; the device writes the hashes
+// into host-mapped memory, so the call's one wait also brings them back.
 int32_t scatter(pa_kv_cache* c, int layer, const std::vector<int64_t>& slots, const void* k,
                 const void* v, hipStream_t stream) {
-  std::map<int64_t, std::vector<int32_t>> by_block;  // block -> token indices, in order
-  for (size_t t = 0; t < slots.size(); ++t) by_block[slots[t] / pa::kBlock].push_back((int32_t)t);
-  const int tasks = (int)by_block.size();
   const int T = (int)slots.size();
-  // one upload: slots (int64 [T]), hashes (uint64 [T], written on the
-  // device), then the int32 task arrays
-  const size_t n32 = (size_t)tasks + (tasks + 1) + 2 * (size_t)T;
-  std::vector<int64_t> host(2 * (size_t)T + (n32 + 1) / 2);
-  // The scatter writes every slot once, from the last token that names it
-  // (the reference writes token by token, so the last one wins; a slot
-  // named twice in one scatter would be unspecified): earlier ones are -1.
-  {
-    std::unordered_set<int64_t> seen;
-    seen.reserve(2 * (size_t)T);
-    for (int t = T - 1; t >= 0; --t) host[t] = seen.insert(slots[t]).second ? slots[t] : -1;
+  int32_t rc = c->ensure_hash_slots(T);
+  if (rc != PA_OK) return rc;
+  // one upload: slots (int64 [T]), then the int32 task arrays (at most T tasks)
+  rc = c->ensure_stage((size_t)T * sizeof(int64_t) + (4 * (size_t)T + 1) * sizeof(int32_t));
+  if (rc != PA_OK) return rc;
+  c->block_task.resize(c->num_blocks, -1);
+  c->task_slots.clear();
+  c->task_slots.reserve(std::min(T, c->num_blocks));  // nothing throws with the table in use
+  auto* slot = (int64_t*)c->host_stage;
+  auto* blk = (int32_t*)(slot + T);
+  int tasks = 0;
+  for (int t = 0; t < T; ++t) {
+    int32_t& task = c->block_task[slots[t] / pa::kBlock];
+    if (task < 0) {
+      c->task_slots.push_back({0, 0});
+      blk[tasks] = (int32_t)(slots[t] / pa::kBlock);
+      task = tasks++;
+    }
+    ++c->task_slots[task].next;
   }
-  auto* i32 = reinterpret_cast<int32_t*>(host.data() + 2 * T);
-  int32_t* blk = i32;
   int32_t* beg = blk + tasks;
   int32_t* tok = beg + tasks + 1;
   int32_t* off = tok + T;
-  int w = 0, i = 0;
-  for (const auto& kv : by_block) {
-    blk[w] = (int32_t)kv.first;
-    beg[w] = i;
-    for (int32_t t : kv.second) {
-      tok[i] = t;
-      off[i] = (int32_t)(slots[t] % pa::kBlock);
-      ++i;
-    }
-    ++w;
+  beg[0] = 0;
+  for (int w = 0; w < tasks; ++w) {
+    beg[w + 1] = beg[w] + c->task_slots[w].next;
+    c->task_slots[w].next = beg[w + 1];
   }
-  beg[tasks] = i;
-  int32_t rc = PA_OK;
-  auto* d = (char*)c->upload(host.data(), host.size() * sizeof(int64_t), stream, &rc);
+  // From the last token backwards: each takes its task's last free place, and
+  // the scatter writes every slot once, from the last token that names it
+  // (the reference writes token by token, so the last one wins; a slot named
+  // twice in one scatter would be unspecified): earlier ones are -1.
+  for (int t = T - 1; t >= 0; --t) {
+    auto& task = c->task_slots[c->block_task[slots[t] / pa::kBlock]];
+    const int o = (int)(slots[t] % pa::kBlock);
+    slot[t] = task.written >> o & 1 ? -1 : slots[t];
+    task.written |= 1u << o;
+    tok[--task.next] = t;
+    off[task.next] = o;
+  }
+  for (int w = 0; w < tasks; ++w) c->block_task[blk[w]] = -1;
+  auto* d = (const char*)c->upload((size_t)((const char*)(off + T) - (const char*)slot), stream,
+                                   &rc);
   if (rc != PA_OK) return rc;
   const auto* d_slots = (const int64_t*)d;
-  auto* d_hash = (uint64_t*)(d + (size_t)T * sizeof(int64_t));
-  const auto* d32 = (const int32_t*)(d + 2 * (size_t)T * sizeof(int64_t));
-  const int32_t *d_blk = d32, *d_beg = d32 + tasks, *d_tok = d_beg + tasks + 1, *d_off = d_tok + T;
+  const auto* d_blk = (const int32_t*)(d + (size_t)T * sizeof(int64_t));
+  const int32_t *d_beg = d_blk + tasks, *d_tok = d_beg + tasks + 1, *d_off = d_tok + T;
   if (c->quantized) {
     rc = pa::launch_quant_write((float*)c->key[layer], (float*)c->value[layer], c->scales[layer],
                                 (const float*)k, (const float*)v, c->num_heads, c->head_dim,
-                                tasks, d_blk, d_beg, d_tok, d_off, d_hash, stream);
+                                tasks, d_blk, d_beg, d_tok, d_off, c->hash_dev, stream);
   } else {
     rc = pa::launch_block_hash_replay(c->key[layer], k, c->dtype, c->num_heads, c->head_dim,
-                                      tasks, d_blk, d_beg, d_tok, d_off, d_hash, stream);
+                                      tasks, d_blk, d_beg, d_tok, d_off, c->hash_dev, stream);
     if (rc == PA_OK)
       rc = pa_reshape_and_cache(k, v, c->key[layer], c->value[layer], d_slots, T, c->num_heads,
                                 c->head_dim, c->num_blocks, 0, 0, c->dtype, (pa_stream_t)stream);
   }
   rc = finish(stream, rc);
   if (rc != PA_OK) return rc;
-  std::vector<uint64_t> hashes(T);
-  if (hipMemcpy(hashes.data(), d_hash, (size_t)T * sizeof(uint64_t), hipMemcpyDeviceToHost) !=
-      hipSuccess) {
-    pa::set_error("pa_kv_cache: reading the block hashes back failed");
-    return PA_ERR_HIP;
-  }
+  const auto* hashes = (volatile uint64_t*)c->hash_host;
   auto& map = c->block_hashes[layer];
-  for (int t = 0; t < T; ++t) map[hashes[t]] = slots[t] / pa::kBlock;
+  for (int t = 0; t < T; ++t) map[(uint64_t)hashes[t]] = slots[t] / pa::kBlock;
   return PA_OK;
 }
 
@@ -286,7 +305,7 @@ extern "C" int32_t pa_kv_cache_write_kv(pa_kv_cache* c, int32_t layer, int64_t b
   hipStream_t s = (hipStream_t)stream;
   if (!c->quantized) {
     // one launch: the block's hash after the token, then the token's rows
-    int32_t rc = c->ensure_hash_slot();
+    int32_t rc = c->ensure_hash_slots(1);
     if (rc != PA_OK) return rc;
     rc = pa::launch_write_token(c->key[layer], c->value[layer], k, v, c->dtype, c->num_heads,
                                 c->head_dim, block_id, (int)token_offset, c->hash_dev, s);
@@ -387,7 +406,10 @@ extern "C" int32_t pa_kv_cache_read_kv(pa_kv_cache* c, int32_t layer, const int6
     if (rc == PA_OK) *n_read = n;
     return rc;
   }
-  void* d_ids = c->upload(ids.data(), ids.size() * sizeof(int32_t), s, &rc);
+  rc = c->ensure_stage(ids.size() * sizeof(int32_t));
+  if (rc != PA_OK) return rc;
+  std::memcpy(c->host_stage, ids.data(), ids.size() * sizeof(int32_t));
+  void* d_ids = c->upload(ids.size() * sizeof(int32_t), s, &rc);
   if (rc != PA_OK) return rc;
   if (c->quantized)
     rc = pa::launch_quant_read((const float*)c->key[layer], (const float*)c->value[layer],
