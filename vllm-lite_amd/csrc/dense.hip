@@ -45,62 +45,123 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(T* __restrict__ out, T* _
     Elem<T>::store(o + i, Elem<T>::load(x + i) * inv * Elem<T>::load(w + i));
 }
 
-// bf16 rows of hidden % 8 == 0, hidden <= 64 * 8 * kNormChunks: one wavefront
-// per row (4 rows per workgroup), the row held in registers as 16-byte
-// chunks (chunk i of lane l is chunk l + 64 i of the row), so x is read once
-// and written at most once; the sum of squares reduced by lane shuffles.
-// Same results as rms_norm_kernel up to the order of the f32 sum.
+// The sum over a row's G lanes: by lane shuffles, and for a workgroup per row
+// over its four wavefronts in LDS.
+template <int G>
+__device__ inline float row_sum(float v, float* red) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  if constexpr (G == 256) {
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = (red[0] + red[1]) + (red[2] + red[3]);
+  }
+  return v;
+}
+
+// RMSNorm (kLayer false) and LayerNorm of rows that are a whole number of
+// 16-byte chunks, at most kNormChunks G of them, all pointers 16-byte aligned:
+// G = 64 lanes (four rows per workgroup) or 256 per row, the row held in
+// registers (chunk i of lane l is chunk l + G i of the row), so x is read once
+// and written at most once, in 16-byte accesses.  Same results as
+// rms_norm_kernel and layer_norm_kernel up to the order of the f32 sums.
+// Bound by a row's latency at small counts and by memory at large ones.
+// Measured against one workgroup per row reading it element by element two or
+// three times (those kernels, kept for other widths and addresses): bf16 RMS
+// 2048 x 4096 22.3 -> 10.1 us, 40 x 4096 9.9 -> 3.4; bf16 layer 8116 x 896
+// 33.2 -> 10.7, 40 x 4096 12.9 -> 4.1; f32 RMS 2048 x 4096 27.3 -> 19.8, layer
+// 35.3 -> 19.5 (6.9 TB/s).
 constexpr int kNormChunks = 4;
-__global__ __launch_bounds__(256) void rms_norm_rows_kernel(uint16_t* __restrict__ out,
-                                                           uint16_t* __restrict__ res,
-                                                           const uint16_t* __restrict__ add,
-                                                           const uint16_t* __restrict__ w,
-                                                           int rows, int hidden, float eps) {
-  const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (row >= rows) return;
-  const int nch = hidden / 8;
-  uint16_t* x = res + row * hidden;
-  const uint16_t* a = add ? add + row * hidden : nullptr;
-  bf16x8 v[kNormChunks], av[kNormChunks];
+template <typename T, int G, bool kLayer>
+__global__ __launch_bounds__(256) void norm_rows_kernel(T* out, T* res, const T* __restrict__ add,
+                                                        const T* __restrict__ w,
+                                                        const T* __restrict__ bias, int rows,
+                                                        int hidden, float eps) {
+  constexpr int E = 16 / sizeof(T);
+  using S = std::conditional_t<sizeof(T) == 2, __bf16, float>;
+  typedef S Chunk __attribute__((ext_vector_type(E)));
+  __shared__ float red[2][4];
+  const int lane = threadIdx.x % G;
+  const int64_t row = (int64_t)blockIdx.x * (256 / G) + threadIdx.x / G;
+  if (row >= rows) return;  // a whole wavefront, or at G = 256 never
+  const int nch = hidden / E;
+  T* x = res + row * hidden;
+  const T* a = add ? add + row * hidden : nullptr;
+  Chunk v[kNormChunks], av[kNormChunks];
 #pragma unroll
   for (int i = 0; i < kNormChunks; ++i) {
-    const int ch = lane + 64 * i;
+    const int ch = lane + G * i;
     if (ch < nch) {
-      v[i] = *reinterpret_cast<const bf16x8*>(x + 8 * ch);
-      if (a) av[i] = *reinterpret_cast<const bf16x8*>(a + 8 * ch);
+      v[i] = *reinterpret_cast<const Chunk*>(x + E * ch);
+      if (a) av[i] = *reinterpret_cast<const Chunk*>(a + E * ch);
     }
   }
-  float ss = 0.f;
+  float sum = 0.f;
 #pragma unroll
   for (int i = 0; i < kNormChunks; ++i) {
-    const int ch = lane + 64 * i;
+    const int ch = lane + G * i;
     if (ch < nch) {
       if (a) {
         // the residual is kept in the storage dtype, as the sum tensor would be
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[i][e] = (__bf16)((float)v[i][e] + (float)av[i][e]);
-        *reinterpret_cast<bf16x8*>(x + 8 * ch) = v[i];
+        for (int e = 0; e < E; ++e) v[i][e] = (S)((float)v[i][e] + (float)av[i][e]);
+        *reinterpret_cast<Chunk*>(x + E * ch) = v[i];
       }
 #pragma unroll
-      for (int e = 0; e < 8; ++e) ss += (float)v[i][e] * (float)v[i][e];
+      for (int e = 0; e < E; ++e) sum += kLayer ? (float)v[i][e] : (float)v[i][e] * (float)v[i][e];
     }
   }
+  sum = row_sum<G>(sum, red[0]);
+  float mean = 0.f;
+  if constexpr (kLayer) {
+    mean = sum / (float)hidden;
+    sum = 0.f;
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
-  const float inv = 1.0f / sqrtf(ss / (float)hidden + eps);
-  uint16_t* orow = out + row * hidden;
+    for (int i = 0; i < kNormChunks; ++i)
+      if (lane + G * i < nch)
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          const float d = (float)v[i][e] - mean;
+          sum += d * d;
+        }
+    sum = row_sum<G>(sum, red[1]);
+  }
+  const float inv = 1.0f / sqrtf(sum / (float)hidden + eps);
+  T* orow = out + row * hidden;
 #pragma unroll
   for (int i = 0; i < kNormChunks; ++i) {
-    const int ch = lane + 64 * i;
+    const int ch = lane + G * i;
     if (ch < nch) {
-      const bf16x8 wv = *reinterpret_cast<const bf16x8*>(w + 8 * ch);
-      bf16x8 r;
+      const Chunk wv = *reinterpret_cast<const Chunk*>(w + E * ch);
+      Chunk bv, r;
+      if (kLayer && bias) bv = *reinterpret_cast<const Chunk*>(bias + E * ch);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) r[e] = (__bf16)((float)v[i][e] * inv * (float)wv[e]);
-      *reinterpret_cast<bf16x8*>(orow + 8 * ch) = r;
+      for (int e = 0; e < E; ++e) {
+        float y = (kLayer ? (float)v[i][e] - mean : (float)v[i][e]) * inv * (float)wv[e];
+        if (kLayer && bias) y += (float)bv[e];
+        r[e] = (S)y;
+      }
+      *reinterpret_cast<Chunk*>(orow + E * ch) = r;
     }
   }
+}
+
+// Launches norm_rows_kernel where the rows fit it; false: they do not.
+// A wavefront per row where the row fits its registers, else a workgroup.
+template <typename T, bool kLayer>
+bool launch_norm_rows(void* out, void* res, const void* add, const void* w, const void* bias,
+                      int rows, int hidden, float eps, hipStream_t s) {
+  constexpr int E = 16 / sizeof(T);
+  const auto bits = (uintptr_t)out | (uintptr_t)res | (uintptr_t)add | (uintptr_t)w |
+                    (uintptr_t)bias;
+  if (hidden % E != 0 || hidden > 256 * E * kNormChunks || (bits & 15) != 0) return false;
+  if (hidden <= 64 * E * kNormChunks)
+    norm_rows_kernel<T, 64, kLayer><<<(rows + 3) / 4, 256, 0, s>>>(
+        (T*)out, (T*)res, (const T*)add, (const T*)w, (const T*)bias, rows, hidden, eps);
+  else
+    norm_rows_kernel<T, 256, kLayer><<<rows, 256, 0, s>>>(
+        (T*)out, (T*)res, (const T*)add, (const T*)w, (const T*)bias, rows, hidden, eps);
+  return true;
 }
 
 __device__ inline float block_sum(float v, float* red) {
@@ -852,8 +913,6 @@ constexpr int kGemmKMultiple = 64;  // K the tiled kernel takes: a multiple of t
 
 using namespace pa;
 
-static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
-
 extern "C" int32_t pa_rms_norm(void* out, void* residual, const void* add, const void* weight,
                                int32_t rows, int32_t hidden, float eps, int32_t dtype,
                                pa_stream_t stream) {
@@ -863,12 +922,13 @@ extern "C" int32_t pa_rms_norm(void* out, void* residual, const void* add, const
   if (rows == 0) return PA_OK;
   PA_REQUIRE(out && residual && weight, PA_ERR_INVALID_ARG, "pa_rms_norm: null pointer");
   hipStream_t s = (hipStream_t)stream;
-  if (dtype == PA_DTYPE_BF16 && hidden % 8 == 0 && hidden <= 64 * 8 * kNormChunks &&
-      aligned16(out) && aligned16(residual) && (!add || aligned16(add)) && aligned16(weight))
-    rms_norm_rows_kernel<<<(rows + 3) / 4, 256, 0, s>>>((uint16_t*)out, (uint16_t*)residual,
-                                                        (const uint16_t*)add,
-                                                        (const uint16_t*)weight, rows, hidden, eps);
-  else if (dtype == PA_DTYPE_BF16)
+  if (dtype == PA_DTYPE_BF16
+          ? launch_norm_rows<uint16_t, false>(out, residual, add, weight, nullptr, rows, hidden,
+                                              eps, s)
+          : launch_norm_rows<float, false>(out, residual, add, weight, nullptr, rows, hidden, eps,
+                                           s))
+    return check_launch("pa_rms_norm");
+  if (dtype == PA_DTYPE_BF16)
     rms_norm_kernel<uint16_t><<<rows, 256, 0, s>>>((uint16_t*)out, (uint16_t*)residual,
                                                    (const uint16_t*)add, (const uint16_t*)weight,
                                                    hidden, eps);
@@ -888,6 +948,10 @@ extern "C" int32_t pa_layer_norm(void* out, void* residual, const void* add, con
   if (rows == 0) return PA_OK;
   PA_REQUIRE(out && residual && weight, PA_ERR_INVALID_ARG, "pa_layer_norm: null pointer");
   hipStream_t s = (hipStream_t)stream;
+  if (dtype == PA_DTYPE_BF16
+          ? launch_norm_rows<uint16_t, true>(out, residual, add, weight, bias, rows, hidden, eps, s)
+          : launch_norm_rows<float, true>(out, residual, add, weight, bias, rows, hidden, eps, s))
+    return check_launch("pa_layer_norm");
   if (dtype == PA_DTYPE_BF16)
     layer_norm_kernel<uint16_t><<<rows, 256, 0, s>>>(
         (uint16_t*)out, (uint16_t*)residual, (const uint16_t*)add, (const uint16_t*)weight,
