@@ -366,6 +366,17 @@ __global__ __launch_bounds__(NT == 1 && U == 4 ? 1024 : 512) void linear_skinny_
       if (rot) pos3 = ra.positions[min(m0 + (j >= 2 ? 16 : 0) + c, M - 1)];
     }
   };
+  // The residual rows of the one-stage instance likewise (only the workgroup
+  // that finishes a tile writes it): behind the K loop their round trip cost
+  // 0.35-0.4 us a launch (32 rows: 896 x 896 5.9 -> 5.5 us, 4864 -> 896 11.0 -> 10.5).
+  const bool add_out = (flags & PA_LINEAR_ADD_OUT) != 0;
+  uint64_t prev8[2] = {0, 0};
+  if (EPI == 0 && U == 8 && add_out && wave == 0) {
+#pragma unroll
+    for (int bb = 0; bb < 2; ++bb)
+      prev8[bb] = *reinterpret_cast<const uint64_t*>(
+          out + (int64_t)min(m0 + 16 * bb + c, M - 1) * N + n0 + 4 * j);
+  }
   if constexpr (U == 8) epi_operands();
   if (s0 < s1) load(s0, a[0], b[0]);
   // The rotation angles of batch rows c (bb 0) and 16 + c (bb 1), computed
@@ -502,7 +513,6 @@ __global__ __launch_bounds__(NT == 1 && U == 4 ? 1024 : 512) void linear_skinny_
 #pragma unroll
     for (int q = 0; q < 2; ++q) inv[q] = 1.0f / sqrtf(ssum[q] / (float)K + eps);
   }
-  const bool add_out = (flags & PA_LINEAR_ADD_OUT) != 0;
 #pragma unroll
   for (int bb = 0; bb < 2; ++bb) {
     const int m = m0 + 16 * bb + c;
@@ -567,7 +577,7 @@ __global__ __launch_bounds__(NT == 1 && U == 4 ? 1024 : 512) void linear_skinny_
         const int n = n0 + 16 * t + 4 * j;
         uint64_t* dst = reinterpret_cast<uint64_t*>(out + (int64_t)m * N + n);
         uint16_t prev[4];
-        if (add_out) *reinterpret_cast<uint64_t*>(prev) = *dst;
+        if (add_out) *reinterpret_cast<uint64_t*>(prev) = EPI == 0 && U == 8 ? prev8[bb] : *dst;
         uint16_t o4[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
