@@ -20,15 +20,17 @@ _DT_BACK = {v: k for k, v in _DTYPES.items()}
 
 def _i64_array(xs):
     # array takes a list of integers in a quarter of the time of int() and
-    # ctypes' conversion (1000 entries: 120 -> 29 us); what it does not take
-    # (floats, numbers as text, more than 64 bits) goes through them.
+    # ctypes' conversion (1000 entries: 120 -> 29 us, even at 4); what it does
+    # not take (floats, numbers as text, more than 64 bits) goes through them.
     xs = list(xs)
-    try:
-        buf = array("q", xs or [0])
-    except (TypeError, OverflowError):
-        xs = [int(x) for x in xs]
-        return (C.c_int64 * max(len(xs), 1))(*xs), len(xs)
-    return (C.c_int64 * len(buf)).from_buffer(buf), len(xs)
+    if len(xs) >= 4:
+        try:
+            buf = array("q", xs)
+            return (C.c_int64 * len(buf)).from_buffer(buf), len(buf)
+        except (TypeError, OverflowError):
+            pass
+    xs = [int(x) for x in xs]
+    return (C.c_int64 * max(len(xs), 1))(*xs), len(xs)
 
 
 class PagedKvCache:
