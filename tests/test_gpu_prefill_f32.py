@@ -96,3 +96,32 @@ def test_block_scales(pa, d):
     s = scales.double()[:, None, None, None]
     ref = reference(q, k.double() * s, v.double() * s, tables, q_lens, past, d ** -0.5)
     assert (out.double() - ref).abs().max() <= 2e-5
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("scale", [math.inf, -math.inf, math.nan])
+def test_block_scale_above_the_diagonal(pa, d, scale):
+    """A block's scale that is not finite (what a quantised write of an infinite
+    value leaves) reaches the rows that attend the block and no earlier one,
+    also where a 16-row tile straddles blocks; the scale of block 0 reaches no
+    row through an id outside the pool."""
+    q_lens, past = [40], [9]
+    q, k, v, tables = case(11, 6, 2, d, q_lens, past)
+    k, v = (k * 40).round().clamp(-127, 127), (v * 40).round().clamp(-127, 127)
+    scales = torch.full((k.shape[0],), 0.02)
+    s = scales.double()[:, None, None, None]
+    ref = reference(q, k.double() * s, v.double() * s, tables, q_lens, past, d ** -0.5)
+    bad = scales.clone()
+    bad[tables[0][2]] = scale  # keys 32 .. 47: rows 23 .. 38
+    out = run(pa, q, k, v, tables, q_lens, past, block_scales=bad.cuda())
+    assert (out[:23].double() - ref[:23]).abs().max() <= 2e-5
+    assert torch.isnan(out[23:]).all()
+    # the pool's block 0 in no table, its scale not finite, one id outside the pool
+    k, v = (torch.cat([torch.zeros_like(t[:1]), t]) for t in (k, v))
+    tables = [[b + 1 for b in t] for t in tables]
+    bad = torch.cat([torch.tensor([scale]), scales])
+    tables[0][1] = -1  # keys 16 .. 31 absent
+    out = run(pa, q, k, v, tables, q_lens, past, block_scales=bad.cuda())
+    assert torch.isfinite(out).all()
+    full = run(pa, q, k, v, tables, q_lens, past, block_scales=torch.cat([scales[:1], scales]).cuda())
+    assert torch.equal(out, full)

@@ -1115,6 +1115,20 @@ __global__ __launch_bounds__(512) void prefill_f32_kernel(
         l += p[b][r];
         p[b][r] *= bscale[b];
       }
+    float odd_scale = 0.f;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) odd_scale += bscale[b] - bscale[b];
+    if (odd_scale != 0.f) {
+      // A masked key's probability stays 0 also where its block's scale is not
+      // finite (0 * inf would reach the rows below the block).
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int t = 4 * j + r;
+          if (t >= lim[b] || (ib + b) * kBlock + t > row_pos) p[b][r] = 0.f;
+        }
+    }
     if (partial) {
       // cache contents past the context may be any bits
 #pragma unroll
