@@ -15,16 +15,18 @@ namespace {
 // out in assembly: with the builtin the compiler cannot tell that the operand
 // reads which follow use another LDS buffer, and makes them wait for the copy
 // (vmcnt(0) right after every copy).  The kernel orders copies and reads
-// itself (wait_copies and a barrier at the top of every step).
+// itself (wait_copies and a barrier at the top of every step).  A load to LDS
+// needs one wait state after the write of m0, which the compiler does not add
+// inside assembly: the s_nop.
 #pragma clang diagnostic ignored "-Winline-asm"  // m0 as a clobber
 __device__ inline void lds_copy16(const uint8_t* base, uint32_t off, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                :
                : "v"(off), "s"(base), "s"(lds)
                : "memory", "m0");
 }
 __device__ inline void lds_copy16(const uint8_t* base, uint64_t off, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off"
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
                :
                : "v"(base + off), "s"(lds)
                : "memory", "m0");
