@@ -63,3 +63,20 @@ def test_reads(pa, dtype, h, d, tokens):
     short = max(1, tokens - 7)
     rk, rv = cache.read_kv(0, ids, short)
     assert torch.equal(rk, k[:short]) and torch.equal(rv, v[:short])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("blocks", [17, 256, 257])
+def test_long_reads_return_complete(pa, dtype, blocks):
+    """A read of more than 16 blocks returns after its stream has run it, so
+    its rows can be used on any stream."""
+    cache = pa.PagedKvCache(1, 1, 64, blocks, dtype)
+    k = torch.randn(blocks * 16, 1, 64).to(dtype).cuda()
+    cache.write_prefill_kv(0, list(range(blocks)), list(range(blocks * 16)), blocks * 16, k, -k)
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        cache.read_kv(0, list(range(blocks)), blocks * 16)  # the outputs' memory is there
+        torch.cuda._sleep(100_000_000)
+        rk, rv = cache.read_kv(0, list(range(blocks)), blocks * 16)
+        assert s.query()
+    assert torch.equal(rk, k) and torch.equal(rv, -k)

@@ -400,9 +400,11 @@ extern "C" int32_t pa_kv_cache_read_kv(pa_kv_cache* c, int32_t layer, const int6
   hipStream_t s = (hipStream_t)stream;
   int32_t rc = PA_OK;
   if (!c->quantized && used <= pa::kSmallIds) {
-    // the ids go in the kernel arguments: no upload, so nothing to wait for
+    // the ids go in the kernel arguments: no upload.  Only the shortest reads
+    // return before the stream has run them (as the header says).
     rc = pa::launch_read_kv_small(c->key[layer], c->value[layer], c->dtype, ids.data(), used, n,
                                   c->num_heads, c->head_dim, c->num_blocks, out_k, out_v, s);
+    if (used > pa::kFewIds) rc = finish(s, rc);
     if (rc == PA_OK) *n_read = n;
     return rc;
   }

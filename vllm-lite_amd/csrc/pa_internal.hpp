@@ -28,7 +28,8 @@ PA_HIDDEN int32_t launch_write_token(void* k_cache, void* v_cache, const void* k
                                      int off, uint64_t* hash_out, hipStream_t stream);
 // read_kv of at most kSmallIds blocks with the ids in the kernel arguments.
 constexpr int kSmallIds = 256;  // 1 KB of the 4 KB of arguments
-constexpr int kFewIds = 16;     // up to these 64 bytes, so a short read does not carry 1 KB
+constexpr int kFewIds = 16;     // up to these 64 bytes, so a short read does not carry 1 KB;
+                                // longer ones return after the stream has run them
 PA_HIDDEN int32_t launch_read_kv_small(const void* k_cache, const void* v_cache, int32_t dtype,
                                        const int32_t* ids, int n_ids, int seq_len, int H, int D,
                                        int num_blocks, void* out_k, void* out_v,
