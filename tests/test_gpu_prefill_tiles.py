@@ -121,3 +121,41 @@ def test_invalid_blocks_first(pa, hq, hkv):
     check(pa, 3, hq, hkv, 128, [70, 5], [40, 90], bad=[(0, 0), (0, 1), (1, 2), (1, 3)], shift=1.5)
     check(pa, 4, hq, hkv, 128, [400] * 12, [0] * 12, bad=[(2, 0), (2, 1), (5, 2), (5, 3)],
           shift=1.5)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("shift", [0.0, 40.0])
+@pytest.mark.parametrize("hq,hkv,d,copies", [(8, 2, 128, 1), (14, 2, 64, 1), (32, 8, 128, 12),
+                                             (14, 2, 64, 30), (32, 8, 128, 40), (14, 2, 64, 110)])
+def test_absent_keys_change_nothing(pa, hq, hkv, d, copies, shift, fp8):
+    """A table that begins with a whole tile (64 keys) of ids outside the pool
+    gives the bits of the table without them: its first present keys are
+    scored as any sequence's first keys are, also far below zero (shift 40:
+    scores of about -18000)."""
+    g = torch.Generator().manual_seed(copies)
+    q_lens = [1 + (37 * i + 69) % 211 for i in range(copies)]
+    past = [(53 * i) % 97 for i in range(copies)]
+    blocks = [(n + p + 15) // 16 for n, p in zip(q_lens, past)]
+    nb = sum(blocks)
+    k = torch.randn(nb, hkv, 16, d, generator=g) * 0.7 + shift
+    v = torch.randn(nb, hkv, d, 16, generator=g)
+    q = (torch.randn(sum(q_lens), hq, d, generator=g) - shift).to(torch.bfloat16).cuda()
+    if fp8:
+        # (code 0x80, torch's -0, is the format's NaN)
+        k, v = (torch.where(t.abs() < 2.0 ** -6, 0.0, t).clamp(-200, 200)
+                .to(torch.float8_e4m3fn).view(torch.uint8) for t in (k, v))
+    else:
+        k, v = k.to(torch.bfloat16), v.to(torch.bfloat16)
+    k, v = k.cuda(), v.cuda()
+    tables = torch.zeros(copies, max(blocks), dtype=torch.int32)
+    o = 0
+    for i, n in enumerate(blocks):
+        tables[i, :n] = torch.arange(o, o + n)
+        o += n
+    cu = torch.tensor([0] + torch.tensor(q_lens).cumsum(0).tolist(), dtype=torch.int32).cuda()
+    pl = torch.tensor(past, dtype=torch.int32)
+    absent = torch.tensor([-1, nb, nb + 7, -5], dtype=torch.int32).expand(copies, 4)
+    outs = [pa.prefill(q, k, v, t.cuda(), cu, p.cuda(), max(q_lens), scale=d ** -0.5)
+            for t, p in ((tables, pl), (torch.cat([absent, tables], 1), pl + 64))]
+    assert outs[0].float().abs().sum() > 0
+    assert torch.equal(outs[0], outs[1])

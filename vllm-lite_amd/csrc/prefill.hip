@@ -28,7 +28,6 @@ namespace {
 
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kNegBig = -1.0e30f;
-constexpr float kNoMax = 16384.f;  // minus the "max" of a row without keys so far (log2 domain)
 
 __device__ inline float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ inline float shfl_xor_f(float x, int mask) { return __shfl_xor(x, mask, 64); }
@@ -699,6 +698,7 @@ __global__ __launch_bounds__(64 * W) void prefill_tiled_kernel(
   f32x4 o[NT][DT];
   f32x4 lacc[NT];  // softmax denominators, accumulated on the matrix core
   float nm[NT];  // minus the rows' running maxima (the Sᵀ accumulators start at it)
+  float raise = 8.0f;  // a score this far above its row's max raises the max
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
     const bool ok = rows_active && r0 + 16 * nt + c < qlen;
@@ -820,27 +820,32 @@ __global__ __launch_bounds__(64 * W) void prefill_tiled_kernel(
         const float t0 = max3_raw(S[nt][0][0], S[nt][0][1], S[nt][0][2]);
         const float t1 = max3_raw(S[nt][0][3], S[nt][1][0], S[nt][1][1]);
         lm[nt] = max3_raw(t0, t1, max3_raw(S[nt][1][2], S[nt][1][3], S[nt][1][3]));
-        need |= lm[nt] > 8.0f;
+        need |= lm[nt] > raise;
       }
       // Rows keep a stale max until one of their scores exceeds it by 2^8;
       // only then is the exact max formed across the four lanes of the row
-      // and the accumulator rescaled.  The first step always sets the max
-      // (m starts at 0, which says nothing about the row's scores).
+      // and the accumulator rescaled.  A row's first step with keys always
+      // sets the max (m starts at 0, which says nothing about the row's
+      // scores): step 0 or, where ids outside the pool masked all of the row's
+      // keys so far, the first with any score (the row's denominator is still
+      // 0 there, and at least 1 from then on).
       const bool first = (KG == 2 || STC == 0) && kt == 0;
-      if (first || __builtin_amdgcn_ballot_w64(need)) {
+      if (__builtin_expect(first || __builtin_amdgcn_ballot_w64(need) != 0, 0)) {
+        raise = 8.0f;
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
           float bm = lm[nt];
           bm = fmaxf(bm, shfl_xor_f(bm, 16));
           bm = fmaxf(bm, shfl_xor_f(bm, 32));
-          // a row with every key of the first step masked starts from a max
-          // so low that its first key exceeds it
-          const float delta = first ? (bm > -INFINITY ? bm : -kNoMax) : fmaxf(bm, 0.f);
+          const bool none = first || lacc[nt][0] == 0.f;
+          const bool masked = !(bm > -INFINITY);
+          if (none && masked) raise = -INFINITY;
+          const float delta = none ? (masked ? 0.f : bm) : fmaxf(bm, 0.f);
           nm[nt] -= delta;
 #pragma unroll
           for (int i = 0; i < 8; ++i) S[nt][i >> 2][i & 3] -= delta;
           if (!first) {
-            const float a = fast_exp2(-delta);
+            const float a = none ? 1.f : fast_exp2(-delta);
             lacc[nt] *= a;
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt) o[nt][dt] *= a;
