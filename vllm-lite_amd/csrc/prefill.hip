@@ -1121,8 +1121,9 @@ __global__ __launch_bounds__(512) void prefill_f32_kernel(
         p[b][r] *= bscale[b];
       }
     float odd_scale = 0.f;
+    if (kv_scales)
 #pragma unroll
-    for (int b = 0; b < NB; ++b) odd_scale += bscale[b] - bscale[b];
+      for (int b = 0; b < NB; ++b) odd_scale += bscale[b] - bscale[b];
     if (odd_scale != 0.f) {
       // A masked key's probability stays 0 also where its block's scale is not
       // finite (0 * inf would reach the rows below the block).
