@@ -223,7 +223,12 @@ size_t pa_decode_workspace_size(int32_t num_seqs, int32_t num_heads, int32_t hea
  *                 its rows, and nothing outside out and the workspace is
  *                 written
  *   scale         softmax scale, e.g. attn_factor / sqrt(D)
- *   workspace     pa_decode_workspace_size() bytes (may be NULL if 0)
+ *   workspace     pa_decode_workspace_size() bytes (may be NULL if 0).  Any
+ *                 call that is given one may write it, also where it could
+ *                 do without (a short context over few sequences is split
+ *                 over more workgroups if the partial results fit), so calls
+ *                 that may overlap need workspaces of their own, and the
+ *                 order of the f32 sums may depend on workspace_bytes
  * out[s, h] = softmax(scale * q[s, h] · K[s, h/g]ᵀ) · V[s, h/g].
  * A table entry outside [0, num_blocks) contributes no keys (its 16
  * positions are masked); the reference would fail on such an id instead
@@ -267,8 +272,8 @@ int32_t pa_decode_fp8_flagged(void* out, const void* q, const void* k_cache, con
  * call).  Sizes whose split needs more (pa_decode_workspace_size() bounds
  * it) return PA_ERR_WORKSPACE without launching.  The stream must belong to
  * the calling thread's current device (PA_ERR_INVALID_ARG otherwise).  Calls
- * on one GPU share the array: calls that may overlap (other streams, other
- * threads) race. */
+ * on one GPU share the array, those over short contexts too: calls that may
+ * overlap (other streams, other threads) race. */
 int32_t pa_decode_noalloc(void* out, const void* q, const void* k_cache, const void* v_cache,
                           const int32_t* block_tables, int32_t max_blocks_per_seq,
                           const int32_t* context_lens, int32_t max_context_len,

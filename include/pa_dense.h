@@ -90,9 +90,12 @@ enum { PA_LINEAR_RMS_IN = 1, PA_LINEAR_ADD_OUT = 2 };
  *    workspace is not used);
  *  - rows > 64 (prompt chunks), or an N the skinny tiles do not divide, with
  *    row-major weights, no PA_LINEAR_RMS_IN and K a multiple of 64: a tiled
- *    GEMM on the matrix cores (128 x 128 output tiles, K staged through LDS
- *    in steps of 64; any N, with SwiGLU a multiple of 64; the workspace is
- *    not used).
+ *    GEMM on the matrix cores (six tilings from 64 x 64 to 256 x 256 output
+ *    tiles, chosen from rows, N and K; K staged through LDS in steps of 64
+ *    or 128; any N, with SwiGLU a multiple of 64; the workspace is not used).
+ *    Some tilings sum K in two or four interleaved parts, so the order of a
+ *    row's f32 sums, and with it the last bit of an output, may depend on
+ *    rows, N and K (equal calls give equal bits).
  * Other shapes return PA_ERR_UNSUPPORTED, as does any dtype but bf16. */
 int32_t pa_linear(void* out, const void* x, const void* weight, const void* bias, int32_t rows,
                   int32_t out_features, int32_t in_features, int32_t act, int32_t packed,

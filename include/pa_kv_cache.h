@@ -14,8 +14,8 @@
  *
  * Unlike the stateless entry points of pa.h, the cache allocates: the
  * caches themselves at creation, a small device staging buffer for block
- * ids / slots, grown on demand, and one host-mapped word for a single
- * token's block hash.  Index arguments marked "host" are read on the host
+ * ids / slots and host-mapped words for the block hashes of one call's
+ * tokens, both grown on demand.  Index arguments marked "host" are read on the host
  * and validated before anything is enqueued.  Writes return after the
  * stream has run them (their block hashes come back to the host), and so
  * does a read_kv over more than 16 blocks or from a quantised cache; a

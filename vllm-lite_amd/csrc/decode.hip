@@ -1575,15 +1575,18 @@ int num_partitions(int max_ctx, int part_len) {
 // Small batches of short contexts (fewer than 512 items at 256 tokens, at
 // most 1024 tokens) take 128-token partitions, up to 8 per (kv head,
 // sequence), which one workgroup merges in LDS.
+// FP8 contexts of two partitions or more, and bf16 ones of up to eight (four
+// at head_dim 256), are taken by workgroups (choose_splits) whose wavefronts
+// share them equally (token_range).  There the length only sets how many
+// wavefronts a workgroup has, but for one workgroup's 128-token partitions.
 int choose_partition(int num_seqs, int num_kv_heads, int max_ctx, int head_dim, int elem_bytes) {
   const long long units = (long long)num_seqs * num_kv_heads;
   auto items = [&](int p) { return units * ((max_ctx + p - 1) / p); };
   // bf16, 1024 tokens: the config-2 shape then has 2048 wavefronts (four
   // partitions merged per workgroup); measured 159.6-159.9 us against
   // 160.4-160.8 at 2048 tokens.  FP8 (four wavefronts per SIMD, one step in
-  // flight each), 512 tokens: 4096 wavefronts, every one resident at once;
-  // past 4096 tokens 1024, so that one workgroup still merges a sequence's
-  // partitions (eight at most) and no reduce launch is needed.
+  // flight each), 512 tokens: 4096 wavefronts, every one resident at once
+  // (past 4096 tokens both lengths give workgroups of eight wavefronts).
   const int long_part = elem_bytes == 1 && max_ctx <= 4096 ? 512 : 1024;
   if (max_ctx <= 8192 && items(long_part) >= 1024) return long_part;
   if (items(512) >= 1024) return 512;

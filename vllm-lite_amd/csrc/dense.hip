@@ -903,7 +903,7 @@ __global__ __launch_bounds__(kArgmaxThreads) void argmax_kernel(int64_t* __restr
 
 constexpr int kSkinnyMaxRows = 64;
 // Compute units of the current device (cached per device).
-int gemm_compute_units() {
+int compute_units() {
   static int cached[64] = {0};
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
@@ -1101,7 +1101,7 @@ extern "C" int32_t pa_linear(void* out, const void* x, const void* weight, const
     // 2 or 1 through three (the LM head back to back: 55-56 us; two
     // 4-wavefront workgroups per CU 57-58 us; three buffers of 7 steps 58)
     auto launch_wide = [&](auto uc, auto nbc) {
-      const int grid = std::min(gemm_compute_units(), (out_features / 16 + 7) / 8);
+      const int grid = std::min(compute_units(), (out_features / 16 + 7) / 8);
       linear_wide_kernel<decltype(uc)::value, decltype(nbc)::value, 8>
           <<<grid, 512, lds, (hipStream_t)stream>>>(
           (uint16_t*)out, (const uint16_t*)x, (const uint16_t*)weight, rows, out_features,
