@@ -343,6 +343,10 @@ extern "C" int32_t pa_batch_attention(pa_batch* b, pa_kv_cache* cache, int32_t l
                "pa_batch_attention: context %d exceeds the capacity %d", b->max_ctx,
                b->capacity);
     const int max_ctx = b->capacity > 0 ? b->capacity : b->max_ctx;
+    // Contexts grow towards the capacity: the launch is planned for three
+    // quarters of it (planned for all of it, 24 layers of 32 sequences of 320 to
+    // 768 tokens took 20 us more per step than in one workgroup each).
+    const int usual_ctx = b->capacity > 0 ? b->capacity - b->capacity / 4 : 0;
     const size_t need = std::max<size_t>(
         pa_decode_workspace_size(b->num_seqs, num_heads, d, max_ctx), 256);
     if (need > b->workspace.bytes) {
@@ -357,7 +361,7 @@ extern "C" int32_t pa_batch_attention(pa_batch* b, pa_kv_cache* cache, int32_t l
       if ((rc = b->workspace.ensure(need))) return rc;
     }
     return pa::decode_strided(out, q, q_stride, kc, vc, (const int32_t*)b->tables.ptr,
-                              b->max_blocks, (const int32_t*)b->ctx_lens.ptr, max_ctx,
+                              b->max_blocks, (const int32_t*)b->ctx_lens.ptr, max_ctx, usual_ctx,
                               b->num_seqs, num_heads, hkv, d, b->num_blocks, scale,
                               b->workspace.ptr, b->workspace.bytes, dtype, stream);
   }

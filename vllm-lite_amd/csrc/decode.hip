@@ -21,11 +21,10 @@
 //    processed per step (32 = the MFMA K dimension of the P·V product).
 //  * decode_generic_kernel (f32 or bf16, any D <= 512, any group size): a
 //    plain reference-grade kernel, one workgroup per query head.
-#include <algorithm>
-#include <cmath>
 #include <mutex>
 #include <type_traits>
 
+#include "decode_splits.hpp"
 #include "pa_common.hpp"
 #include "pa_internal.hpp"
 
@@ -1594,47 +1593,6 @@ int choose_partition(int num_seqs, int num_kv_heads, int max_ctx, int head_dim, 
   return kPart;
 }
 
-// Workgroups per (kv head, sequence) whose results the reduce kernel merges,
-// for launches whose wavefronts merge in LDS.  One workgroup streams at most
-// about 43 GB/s (bf16; FP8, with one step in flight per wavefront, 36; 36 / 31
-// with 32 of them running, 29 / 25 with 128), so few (kv head, sequence) pairs leave the
-// chip idle, and a number of them that does not fill whole rounds of the 256
-// CUs leaves it idle in the last.  More workgroups cost the reduce launch
-// (3.2 us) and 1.4% of the stream each.  Estimated over the launch's longest
-// context for every sequence (the others' are on the device); the least
-// wins, one workgroup where they tie.  Measured, us, one workgroup / chosen:
-// bf16, 8 kv heads x 128: 1 x 2000 tokens 27.0 / 10.0, 1 x 500 9.8 / 7.5, 4 x
-// 2000 32.1 / 11.3, 16 x 200-2000 27.3 / 19.6, 48 x 4096 157 / 132, 37 x
-// 500-8000 120 / 91, 64 x 4096 170 / 170 (one; two workgroups 175); FP8: 37 x
-// 500-8000 69 / 56, 16 x 8000 78 / 50, 1 x 2000 19 / 9.
-int choose_splits(int num_seqs, int num_heads, int num_kv_heads, int head_dim, int max_ctx,
-                  int elem_bytes, size_t workspace_bytes) {
-  constexpr double kCUs = 256;
-  const double pairs = (double)num_seqs * num_kv_heads;
-  const double pair_us = 2e-3 * max_ctx * head_dim * elem_bytes;  // bytes / 1000: us at 1 GB/s
-  const double all = elem_bytes == 1 ? 6200. : 6500.;
-  auto one = [&](double wgs) {
-    return (elem_bytes == 1 ? 36. : 43.) * (wgs <= 16 ? 1. : wgs <= 64 ? 0.85 : 0.68);
-  };
-  int best = 1;
-  double best_us = 0.;
-  for (int s : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32}) {
-    const double wgs = pairs * s;
-    if (s > 1 && (max_ctx < 64 * s || wgs > 4096. ||
-                  (size_t)num_seqs * num_heads * s * (head_dim + 2) * sizeof(float) >
-                      workspace_bytes))
-      break;
-    const double rounds = wgs <= kCUs ? 1. : std::ceil(wgs / kCUs) * kCUs / wgs;
-    double us = std::max(pairs * pair_us / all * rounds, wgs <= kCUs ? pair_us / s / one(wgs) : 0.);
-    if (s > 1) us = us * (1. + 0.014 * s) + 3.2;
-    if (s == 1 || us < best_us) {
-      best = s;
-      best_us = us;
-    }
-  }
-  return best;
-}
-
 }  // namespace
 }  // namespace pa
 
@@ -1666,7 +1624,7 @@ struct DecodePlan {
 };
 DecodePlan decode_plan(int32_t dtype, bool quantized, int32_t num_seqs, int32_t num_heads,
                        int32_t num_kv_heads, int32_t head_dim, int32_t max_context_len,
-                       size_t workspace_bytes) {
+                       int32_t usual_context_len, size_t workspace_bytes) {
   DecodePlan p{};
   const int G = num_heads / num_kv_heads;
   const bool fp8 = dtype == PA_DTYPE_FP8_E4M3;
@@ -1696,7 +1654,7 @@ DecodePlan decode_plan(int32_t dtype, bool quantized, int32_t num_seqs, int32_t 
   // FP8 contexts of more partitions than that: eight wavefronts share them
   if (fp8 && p.mfma && p.np > 1 && p.merge_waves == 1) p.merge_waves = head_dim <= 128 ? 8 : 4;
   p.splits = p.merge_waves > 1 ? choose_splits(num_seqs, num_heads, num_kv_heads, head_dim,
-                                               max_context_len, fp8 ? 1 : 2, workspace_bytes)
+                                               usual_context_len, fp8 ? 1 : 2, workspace_bytes)
                                : 1;
   // Partitioned launches that need the reduce (long, ragged contexts) cut
   // the work evenly over the GPU instead (bf16 caches).
@@ -1730,7 +1688,7 @@ int32_t decode_impl(void* out, const void* q, const void* k_cache, const void* v
                     int32_t max_context_len, int32_t num_seqs, int32_t num_heads,
                     int32_t num_kv_heads, int32_t head_dim, int32_t num_blocks, float scale,
                     void* workspace, size_t workspace_bytes, int32_t dtype, pa_stream_t stream, int64_t q_row = 0,
-                    const uint8_t* block_flags = nullptr) {
+                    const uint8_t* block_flags = nullptr, int32_t usual_context_len = 0) {
   clear_error();
   PA_REQUIRE(dtype_ok(dtype) || dtype == PA_DTYPE_FP8_E4M3, PA_ERR_INVALID_ARG,
              "pa_decode: unknown dtype %d", dtype);
@@ -1748,6 +1706,7 @@ int32_t decode_impl(void* out, const void* q, const void* k_cache, const void* v
              "pa_decode: null pointer");
   const DecodePlan plan = decode_plan(dtype, kv_scales != nullptr, num_seqs, num_heads,
                                       num_kv_heads, head_dim, max_context_len,
+                                      usual_context_len > 0 ? usual_context_len : max_context_len,
                                       workspace ? workspace_bytes : 0);
   const int G = num_heads / num_kv_heads;
   const bool fp8 = dtype == PA_DTYPE_FP8_E4M3;
@@ -1949,13 +1908,14 @@ namespace pa {
 int32_t decode_strided(void* out, const void* q, int64_t q_row, const void* k_cache,
                        const void* v_cache, const int32_t* block_tables,
                        int32_t max_blocks_per_seq, const int32_t* context_lens,
-                       int32_t max_context_len, int32_t num_seqs, int32_t num_heads,
-                       int32_t num_kv_heads, int32_t head_dim, int32_t num_blocks, float scale,
-                       void* workspace, size_t workspace_bytes, int32_t dtype,
-                       pa_stream_t stream) {
+                       int32_t max_context_len, int32_t usual_context_len, int32_t num_seqs,
+                       int32_t num_heads, int32_t num_kv_heads, int32_t head_dim,
+                       int32_t num_blocks, float scale, void* workspace, size_t workspace_bytes,
+                       int32_t dtype, pa_stream_t stream) {
   return decode_impl(out, q, k_cache, v_cache, nullptr, block_tables, max_blocks_per_seq,
                      context_lens, max_context_len, num_seqs, num_heads, num_kv_heads, head_dim,
-                     num_blocks, scale, workspace, workspace_bytes, dtype, stream, q_row);
+                     num_blocks, scale, workspace, workspace_bytes, dtype, stream, q_row, nullptr,
+                     usual_context_len);
 }
 }  // namespace pa
 
@@ -2014,7 +1974,8 @@ extern "C" int32_t pa_decode_noalloc(void* out, const void* q, const void* k_cac
   if (num_seqs > 0 && num_heads > 0 && num_kv_heads > 0 && head_dim > 0 &&
       num_heads % num_kv_heads == 0 && max_context_len > 0) {
     const DecodePlan plan = decode_plan(dtype, false, num_seqs, num_heads, num_kv_heads,
-                                        head_dim, max_context_len, kDecodeScratchBytes);
+                                        head_dim, max_context_len, max_context_len,
+                                        kDecodeScratchBytes);
     PA_REQUIRE(plan.ws_bytes <= kDecodeScratchBytes, PA_ERR_WORKSPACE,
                "pa_decode_noalloc: %d sequences x %d heads at context %d need %zu bytes of "
                "split-K scratch, above the fixed %zu (use pa_decode with a workspace)",

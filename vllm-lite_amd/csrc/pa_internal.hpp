@@ -46,14 +46,16 @@ PA_HIDDEN int32_t launch_gemm(void* out, const void* x, const void* weight, cons
                               bool add_out, hipStream_t stream);
 
 // pa_decode / pa_prefill with q rows q_row elements apart (a view of a fused
-// QKV projection output); pa_batch_attention's path.
+// QKV projection output); pa_batch_attention's path.  usual_context_len: the
+// length to plan for where max_context_len is a bound far ahead (0: the bound).
 PA_HIDDEN int32_t decode_strided(void* out, const void* q, int64_t q_row, const void* k_cache,
                                  const void* v_cache, const int32_t* block_tables,
                                  int32_t max_blocks_per_seq, const int32_t* context_lens,
-                                 int32_t max_context_len, int32_t num_seqs, int32_t num_heads,
-                                 int32_t num_kv_heads, int32_t head_dim, int32_t num_blocks,
-                                 float scale, void* workspace, size_t workspace_bytes,
-                                 int32_t dtype, hipStream_t stream);
+                                 int32_t max_context_len, int32_t usual_context_len,
+                                 int32_t num_seqs, int32_t num_heads, int32_t num_kv_heads,
+                                 int32_t head_dim, int32_t num_blocks, float scale,
+                                 void* workspace, size_t workspace_bytes, int32_t dtype,
+                                 hipStream_t stream);
 PA_HIDDEN int32_t prefill_strided(void* out, const void* q, int64_t q_row, const void* k_cache,
                                   const void* v_cache, const int32_t* block_tables,
                                   int32_t max_blocks_per_seq, const int32_t* cu_q_lens,
