@@ -1,7 +1,8 @@
 """The tiled RoPE + KV-cache write against the one-token kernel it stands in
-for (which still takes rows that are not 16-byte aligned): equal bit for bit,
-for token counts around the 16-token tiles, runs of slots at every block
-offset, scattered and skipped slots, and every head dim it takes."""
+for (which still takes rows that are not 16-byte aligned, and fewer than 512
+tokens of at most 512 rotation pairs): equal bit for bit, for token counts
+around the 16-token tiles, runs of slots at every block offset, scattered and
+skipped slots, and every head dim it takes."""
 import pytest
 import torch
 
@@ -20,9 +21,11 @@ def slots_of(kind, t, nb, g):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("hq,hkv,d", [(14, 2, 64), (32, 8, 128), (4, 4, 16), (3, 1, 256), (6, 2, 80)])
+@pytest.mark.parametrize("hq,hkv,d", [(14, 2, 64), (32, 8, 128), (4, 4, 16), (3, 1, 256), (6, 2, 80),
+                                      (16, 2, 64), (48, 24, 16), (5, 1, 256), (12, 2, 80)])
 @pytest.mark.parametrize("t,kind", [(1, "scattered"), (15, "3"), (16, "0"), (17, "15"), (40, "scattered"),
-                                    (100, "9"), (333, "0")])
+                                    (100, "9"), (333, "0"), (511, "3"), (512, "scattered"),
+                                    (600, "7")])
 def test_equals_one_token_kernel(pa, dtype, hq, hkv, d, t, kind):
     g = torch.Generator().manual_seed(t + d)
     nb = (t + 47) // 16 + 2

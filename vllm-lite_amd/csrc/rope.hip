@@ -259,9 +259,14 @@ extern "C" int32_t pa_rope_reshape_and_cache(void* q, int64_t q_stride, const vo
              PA_ERR_INVALID_ARG, "pa_rope_reshape_and_cache: token stride too small");
   const int64_t num_slots = (int64_t)num_blocks * kBlock;
   hipStream_t s = (hipStream_t)stream;
-  // 16-byte pieces of every row: aligned bases and strides
+  // 16-byte pieces of every row: aligned bases and strides.  Few tokens of at
+  // most 512 rotation pairs (two per thread) stay with the one-token kernel:
+  // us, one-token / tiled, bf16, 8 / 2 heads x 48: 1 token 2.5 / 3.4, 300 3.1 /
+  // 3.6, 1000 3.7 / 3.8; 14 / 2 x 64: 1 token 3.0 / 3.2, 300 3.6 / 3.4, 1000 4.5 /
+  // 3.7; more heads, 32 / 8 x 80 (1600 pairs): 1 token 4.8 / 3.6.
   const int es = (int)dtype_size(dtype);
-  const bool tiled = head_dim % 16 == 0 && head_dim <= 256 &&
+  const bool few = num_tokens < 512 && (num_heads + num_kv_heads) * (int64_t)head_dim <= 1024;
+  const bool tiled = !few && head_dim % 16 == 0 && head_dim <= 256 &&
                      ((uintptr_t)q | (uintptr_t)key | (uintptr_t)value | (uintptr_t)k_cache |
                       (uintptr_t)v_cache) % 16 == 0 &&
                      (q_stride * es) % 16 == 0 && (key_stride * es) % 16 == 0 &&
