@@ -70,7 +70,7 @@ __device__ inline float row_sum(float v, float* red) {
 // three times (those kernels, kept for other widths and addresses): bf16 RMS
 // 2048 x 4096 22.3 -> 10.1 us, 40 x 4096 9.9 -> 3.4; bf16 layer 8116 x 896
 // 33.2 -> 10.7, 40 x 4096 12.9 -> 4.1; f32 RMS 2048 x 4096 27.3 -> 19.8, layer
-// 35.3 -> 19.5 (6.9 TB/s).
+// 35.3 -> 19.5 (6.9 TB/s, out of the last-level cache).
 constexpr int kNormChunks = 4;
 template <typename T, int G, bool kLayer>
 __global__ __launch_bounds__(256) void norm_rows_kernel(T* out, T* res, const T* __restrict__ add,
