@@ -306,10 +306,10 @@ def test_linear_split_k_workspace_any_call_order(pa):
         torch.testing.assert_close(got.float(), x.float() @ w.float().T, atol=2e-2, rtol=1e-2)
 
 
-# Prefill-sized batches (rows > 64) take the tiled GEMM (gemm_tiled_kernel,
-# 128 x 128 workgroup tiles, or 256 x 256 for outputs of 256 such tiles or
-# more): the config-5 projections at prompt-chunk row counts, ragged row and
-# column tails around both tiles, bias, SwiGLU and the residual add.
+# Prefill-sized batches (rows > 64) take the tiled GEMM (gemm_kernel; its
+# tilings one by one in test_gpu_gemm.py): the config-5 projections at
+# prompt-chunk row counts, ragged row and column tails, bias, SwiGLU and the
+# residual add.
 @pytest.mark.parametrize("m,n,k", [(65, 896, 896), (130, 256, 896), (1000, 896, 896),
                                    (777, 896, 4864), (128, 128, 64), (4100, 1152, 896),
                                    (2100, 8000, 128), (9000, 896, 896)])
